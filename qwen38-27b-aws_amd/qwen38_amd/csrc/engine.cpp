@@ -93,10 +93,12 @@ struct q38_handle {
         off_sp_sin, off_sp_states, off_sp_out, off_sp_current, off_sp_ids, off_sp_at, off_sp_draft, off_gemm, off_gates, off_status,
         workspace_bytes;
     // prefill scratch (with a prefill chunk in the config)
-    size_t off_pqn = 0, off_pkn = 0, off_pv = 0, off_po = 0, off_pbeta = 0, off_pg = 0, off_pqs = 0;
+    size_t off_pqn = 0, off_pkn = 0, off_pv = 0, off_po = 0, off_pbeta = 0, off_pg = 0, off_pqs = 0, off_pmx = 0, off_ppart = 0,
+           off_prows = 0, off_pkw = 0, off_pvw = 0;
     size_t part_floats;  // capacity of the split-K partial buffer
     int gate_groups;  // K ranges of the gated-delta gate projections
     int attn_nchunks;  // chunks of ATTN_CHUNK cached positions over S
+    size_t prefill_slots = 0;  // slots of the prefill attention's partial sums
     size_t attn_pv_floats;  // capacity of the chunked attention's split sums
     // Kernel timer (q38_kernel_timer): event pairs around the gate/up GEMM launches while on.
     std::vector<hipEvent_t> timer_events;
@@ -493,6 +495,12 @@ int run_mixer(q38_handle* h, int li, const StepIO& io, int rd, int wr, hipStream
             p.k_scale = ks;
             p.v_scale = vs;
             p.qs = (uint16_t*)h->ws(h->off_pqs);
+            p.mx = (int*)h->ws(h->off_pmx);
+            p.part = (float*)h->ws(h->off_ppart);
+            p.part_rows = (float*)h->ws(h->off_prows);
+            p.part_slots = h->prefill_slots;
+            p.k_wide = (bf16_t*)h->ws(h->off_pkw);
+            p.v_wide = (bf16_t*)h->ws(h->off_pvw);
             p.act = act_mid;
             p.eps = h->cfg.rms_norm_eps;
             HIP_TRY(q38_attn_prefill(p, stream));
@@ -738,6 +746,14 @@ int q38_create(const q38_config* cfg, q38_handle** out) {
         h->off_pbeta = take(Tc * h->Hv * 4);
         h->off_pg = take(Tc * h->Hv * 4);
         h->off_pqs = take((size_t)h->Hq * Tc * 256 * 2);
+        h->off_pmx = take((size_t)h->Hq * ((h->S + Tc + 2047) / 2048) * Tc * 4);
+        h->prefill_slots = prefill_slots(c.prefill_chunk, h->Hq, h->Hkv);
+        h->off_ppart = take(h->prefill_slots * 4 * 64 * 256 * 4);
+        h->off_prows = take(h->prefill_slots * 256 * 2 * 4);
+        if (c.kv_cache_format == Q38_KV_FP8) {
+            h->off_pkw = take((size_t)h->Hkv * h->S * 256 * 2);
+            h->off_pvw = take((size_t)h->Hkv * h->S * 256 * 2);
+        }
     }
     h->workspace_bytes = o;
     *out = h;

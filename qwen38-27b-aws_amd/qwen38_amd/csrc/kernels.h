@@ -135,7 +135,26 @@ struct PrefillAttnArgs {
     int kv8;                 // e4m3 caches with the layer's scales, as AttnArgs
     const bf16_t* k_scale;
     const bf16_t* v_scale;
+    int* mx;                 // scratch [Hq][blocks of 2048 over S + L][L]: largest score per token and block, as ordered ints
+    float* part;             // scratch [part_slots][4][64][256]: an item's sums of weights x V
+    float* part_rows;        // scratch [part_slots][256][2]: an item's maximum and weight sum per token
+    size_t part_slots;
+    bf16_t* k_wide;          // kv8: scratch [Hkv][S][256], the row's keys widened
+    bf16_t* v_wide;          // kv8: scratch [Hkv][S/32][256][32]
+    const bf16_t* kw;        // set by the launcher: the keys and values the attention reads, and whether they hold every
+    const bf16_t* vw;        // row (the caches) or only this one (the widened copies)
+    int kw_slot, ns_max, cus;
 };
+
+constexpr int PREFILL_RANGES = 8;   // most ranges of positions a prefill attention tile is split into
+constexpr int PREFILL_ITEMS = 768;  // most items in all, when the tiles alone are not more
+// Slots of the prefill attention's partial sums for chunks of up to L tokens: quads * min(PREFILL_RANGES,
+// max(1, PREFILL_ITEMS / quads)) with quads = Hkv * ceil(Hq / Hkv * ceil(L / 64) / 4), at its largest.
+inline size_t prefill_slots(int L, int Hq, int Hkv) {
+    const size_t quads = (size_t)Hkv * ((Hq / Hkv * ((L + 63) / 64) + 3) / 4);
+    const size_t split = quads * PREFILL_RANGES;
+    return quads > PREFILL_ITEMS ? quads : split < PREFILL_ITEMS ? split : (size_t)PREFILL_ITEMS;
+}
 
 #define ATTN_KMAX 8   // verify tokens
 #define ATTN_QMAX 64  // query rows per KV head

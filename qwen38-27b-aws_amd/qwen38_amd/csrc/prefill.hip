@@ -17,13 +17,16 @@
 //   attn_prefill_prep  (token): q and k RMS norms and RoPE in bf16 (model.py:565-577), q times 1/16 (exact) to scratch;
 //                      the chunk's keys and values into row slot's cache at start .. start + L - 1 (model.py:791-799;
 //                      the other rows' junk writes at the cache's end are left out: nothing reads them)
-//   attn_prefill       (128 tokens, query head), four waves of 32 tokens sharing each 32-position K/V sub-block through
-//                      LDS: blocked_attention (model.py:170-191) over the row's cached
+//   attn_prefill_widen an FP8 cache's row widened to bf16 once
+//   attn_prefill_max, attn_prefill, attn_prefill_finish: blocked_attention (model.py:170-191) over the row's cached
 //                      positions before `start` and the chunk's own tokens causally, in the reference's blocks of 2048
 //                      positions of [cache, chunk]: per block the running max, e^(s - max) summed in float32, the
-//                      weights in bf16 times V on the MFMA (float32 sums, rounded to bf16 once per block, as the
-//                      reference's bf16 matmul), output and sum rescaled across blocks; then out / sum, the gate, e5m2.
-//                      Positions a row cannot see are skipped: the reference gives them weights of exactly zero.
+//                      weights in bf16 times V on the MFMA with float32 sums, output and sum rescaled across blocks;
+//                      then out / sum, the gate, e5m2. Positions a row cannot see are skipped: the reference gives them
+//                      weights of exactly zero.
+#include <algorithm>
+#include <type_traits>
+
 #include "kernels.h"
 
 namespace {
@@ -211,16 +214,11 @@ namespace {
 
 constexpr int QP = 256;  // bf16 per scaled query row in the scratch
 
-__device__ __forceinline__ v8bf16 load8p(const bf16_t* p) { return *(const v8bf16*)p; }
-__device__ __forceinline__ int drow(int i, int lane) { return 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3); }
-
-// Direct global -> LDS copy of one dword per lane from base + off (base wave-uniform, in scalar registers): lane l's 4
-// bytes land at LDS address dst + 4 l (dst wave-uniform). Inline assembly, so the compiler neither counts it nor waits
-// for it; the ring's own vmcnt waits below cover it.
-__device__ __forceinline__ void lds_dword(const void* base, uint32_t off, uint32_t dst) {
-    const uint32_t m0 = __builtin_amdgcn_readfirstlane(dst);
-    asm volatile("global_load_lds_dword %0, %1" ::"v"(off), "s"(base), "{m0}"(m0) : "memory");
+__device__ __forceinline__ int order_bits(float f) {  // floats in the order of signed ints
+    const int i = __float_as_int(f);
+    return i >= 0 ? i : i ^ 0x7fffffff;
 }
+__device__ __forceinline__ v8bf16 load8p(const bf16_t* p) { return *(const v8bf16*)p; }
 
 // Wait until at most N of this wave's vector-memory operations are outstanding (its copies into the stage about to be
 // read have landed) and its LDS reads have returned, then meet the other waves: after it the stage read one step
@@ -228,36 +226,6 @@ __device__ __forceinline__ void lds_dword(const void* base, uint32_t off, uint32
 template <int N>
 __device__ __forceinline__ void ring_ready() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-
-// Every LDS read of this wave has returned; then meet the other waves, so the stage just read can be refilled.
-__device__ __forceinline__ void ring_release() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// LDS layout of one 32-position sub-block (E bytes per element), swizzled at the granularity the MFMA operand reads use
-// so that they are free of bank conflicts, and filled by coalesced dword copies (each copy instruction of a wave takes
-// 256 contiguous bytes of the cache, permuted within rows). The maps are their own inverses.
-//   K [32 positions][256 dims]: bf16 16-byte chunk c of row r at chunk c ^ (r & 15); e4m3 8-byte chunk c at c ^ r.
-//   V [256 dims][32 positions]: bf16 8-byte chunk c of row d at c ^ ((d >> 2) & 7); e4m3 4-byte chunk c at
-//   c ^ (((d >> 3) & 3) << 1).
-template <int E>
-__device__ __forceinline__ uint32_t k_swz(uint32_t byte) {  // byte offset in the sub-block, either direction
-    if constexpr (E == 2) {
-        const uint32_t r = byte >> 9;
-        return byte ^ ((r & 15) << 4);
-    } else {
-        const uint32_t r = byte >> 8;
-        return byte ^ ((r & 31) << 3);
-    }
-}
-template <int E>
-__device__ __forceinline__ uint32_t v_swz(uint32_t byte) {
-    if constexpr (E == 2) {
-        const uint32_t d = byte >> 6;
-        return byte ^ (((d >> 2) & 7) << 3);
-    } else {
-        const uint32_t d = byte >> 5;
-        return byte ^ (((d >> 3) & 3) << 3);
-    }
 }
 
 }  // namespace
@@ -313,6 +281,8 @@ __global__ __launch_bounds__(256) void attn_prefill_prep_kernel(const PrefillAtt
             out[e] = d < 64 ? rbf(rbf(hn[e] * cs[e]) + rbf((d < 32 ? -part : part) * sn[e])) : hn[e];
         }
         if (r < Hq) {
+            for (int b = lane; b < (S + a.L + 2047) >> 11; b += 64)  // the row's block maxima start below every score
+                a.mx[((size_t)r * ((S + a.L + 2047) >> 11) + b) * a.L + t] = order_bits(-INFINITY);
             *(uint2*)(a.qs + ((size_t)r * a.L + t) * QP + d0) =
                 make_uint2(pk_bf16(out[0] * 0.0625f, out[1] * 0.0625f), pk_bf16(out[2] * 0.0625f, out[3] * 0.0625f));
         } else if (p < S) {
@@ -327,241 +297,514 @@ __global__ __launch_bounds__(256) void attn_prefill_prep_kernel(const PrefillAtt
     }
 }
 
-// Grid (query head, tiles of 128 tokens), four waves: wave w takes tokens T0 + 32 w .. + 31. The four waves see the
-// same cached positions, so each sub-block of 32 positions is copied into LDS once per workgroup (a ring of three
-// stages: the next two sub-blocks' copies are in flight while the current one is used, one barrier per sub-block) and
-// read by all four.
-// Scores by v_mfma_f32_32x32x16_bf16 with the keys as A (32 positions) and the queries as B (32 tokens): lane l holds
-// token t0 + l % 32 and positions drow(i, l); MFMA step m takes dims 8 m .. 8 m + 7 in lanes 0-31 and 128 + 8 m .. in
-// lanes 32-63 (the queries in the same order). The weights go straight from those registers into the A operand of
-// weights x V (two MFMA steps of 16 positions: rows drow(0..7) and drow(8..15) of the lane), with V's B operand read in
-// the same position order from the transposed sub-block. With KV8 the cached bytes (the chunk's own included, written by
-// the prep kernel) widen to bf16(e4m3 x scale) as they are read from LDS. Every wave runs all of the workgroup's
-// sub-blocks: those past its own tokens (at most three, on the diagonal, where the workgroup waits for its last wave
-// anyway) hold chunk positions the prep kernel wrote, so they add weights of exactly zero times finite values, which
-// leaves the sums as they were (none of them is -0: they start at +0). A block none of a wave's tokens sees leaves
-// its state alone. The output so far stays in registers.
-template <bool KV8>
-__global__ __launch_bounds__(256) void attn_prefill_kernel(const PrefillAttnArgs a) {
-    constexpr int E = KV8 ? 1 : 2;        // bytes per cached element
-    constexpr int SUB = 32 * 256 * E;     // bytes of one K (or V) sub-block
-    constexpr int NCP = SUB / 1024;       // dword copies per wave per sub-block of one array
-    __shared__ __attribute__((aligned(1024))) uint8_t ring[3][2][SUB];  // [stage][K, V]
-    __shared__ float s_row[4][32];
-    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // Workgroups start in the order of their linear id, x fastest, and go to the XCDs in turn: the last (heaviest,
-    // causally) tiles start first, and with 8 | Hq the query heads of one XCD are consecutive (one KV head's, when
-    // G >= Hq / 8), so its L2 holds few KV heads' keys and values.
-    const int T0 = (gridDim.y - 1 - blockIdx.y) * 128;
-    const int hq = a.Hq % 8 ? blockIdx.x : (blockIdx.x % 8) * (a.Hq / 8) + blockIdx.x / 8;
-    const int L = a.L, S = a.S, G = a.Hq / a.Hkv, kvh = hq / G, t0 = T0 + 32 * wv;
-    const int slot = *a.slot, start = *a.start;
-    if (start < 0 || start + L > S || slot < 0 || slot >= a.rows) return;  // the host checks these too
-    const bool live = t0 < L;         // wave-uniform: the wave has tokens
-    const int tq = t0 + (lane & 31);  // this lane's token (query)
-    const size_t head = (size_t)slot * a.Hkv + kvh;
-    const float ksc = KV8 ? bf2f(*a.k_scale) : 0.0f, vsc = KV8 ? bf2f(*a.v_scale) : 0.0f;
-    const uint8_t* kg = (const uint8_t*)a.k_cache + head * S * 256 * E;
-    const uint8_t* vg = (const uint8_t*)a.v_cache + head * S * 256 * E;
-    const uint32_t lds0 = (uint32_t)(uintptr_t)LDS_PTR(&ring[0][0][0]);
+// ---- Attention over one chunk: attn_prefill_max, attn_prefill, attn_prefill_finish.
+//
+// A wave takes 64 tokens of one query head; a workgroup's four waves take four consecutive (64 tokens, query head) tiles
+// of one KV head, heads fastest, so they see nearly the same positions, and each 32-position sub-block of K (and V) is
+// copied into an LDS ring once and read by all four. 64 tokens per wave, because with 32 the waves' reads of the
+// sub-blocks take the LDS as long as their MFMAs take the matrix cores (16 KB per 16 MFMAs and wave, 128 B a cycle).
+// The 64 x 256 output (256 registers), the queries (128) and the scores then fill one wave per SIMD.
+//
+// The weights are the reference's bf16(e^(s - m)), m the running maximum through the end of the block of 2048 that
+// holds the position, so m has to be known before a block's first weight: attn_prefill_max makes one pass over the
+// scores for the blocks' maxima (two waves per SIMD), attn_prefill a second one for weights x V. Since every block's
+// maximum is then known, a tile's positions need not be taken in order by one workgroup: the work is dealt out as items
+// (tile of four waves, range of sub-blocks), as many ranges per tile as fill the CUs evenly (prefill_plan), and
+// attn_prefill_finish adds the ranges' float32 sums in order.
+//
+// Bounds: the matrix cores. 2,048 tokens after 14,336 positions of the 27B layer (24 x 256 dims): 3 x 387 GFLOP in 302 +
+// 892 + 48 us (0.93 PFLOP/s; two passes over the scores), before with 32 tokens a wave, 128 a workgroup and every tile's
+// positions in one workgroup 3,669 us. 416 tokens after 1,111 over an FP8 cache: 95 us (widening, maxima, weights x V
+// and sums), before 267.
+namespace {
 
-    v8bf16 qf[16];
-    if (live) {
-        const bf16_t* qp = a.qs + ((size_t)hq * L + tq) * QP + (lane >> 5) * 128;
-#pragma unroll
-        for (int m = 0; m < 16; ++m) qf[m] = load8p(qp + m * 8);
-    } else {
-#pragma unroll
-        for (int m = 0; m < 16; ++m)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) qf[m][e] = (__bf16)0.0f;
-    }
-    v16f so[8];  // output so far: so[db][i] is token drow(i, l), dim 32 db + l % 32
-#pragma unroll
-    for (int db = 0; db < 8; ++db)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) so[db][i] = 0.0f;
-    float best = 2.0f * -1e4f, total = 0.0f;
+constexpr int PF_ROWS = 64;                  // tokens per wave
+constexpr int PF_SUB = 32 * 256 * 2;         // bytes of one K or V sub-block in LDS
+constexpr float LOG2E = 1.4426950408889634f;
 
-    // This wave's dword copies of the sub-block at p0 into stage st: copy j of lane l fills LDS byte at + 4 l of the
-    // stage, at = 256 (4 j + w), from the cache byte the swizzle maps there. A wave's 256 bytes lie in rows that share
-    // one swizzle (K rows hold 256 or 512 bytes; V rows 64 or 32 bytes, in groups of 4 or 8 with one pattern), so that
-    // byte is at + (4 l ^ X) with X = swz(at) ^ at uniform over the wave.
-    auto copy = [&](int p0, int st, bool with_v) {
-        const uint32_t dst = lds0 + (uint32_t)st * 2 * SUB;
-        const uint8_t* ks = kg + (size_t)p0 * 256 * E;
-#pragma unroll
-        for (int j = 0; j < NCP; ++j) {
-            const uint32_t at = (j * 4 + wv) * 256;
-            lds_dword(ks + at, (uint32_t)(lane * 4) ^ (k_swz<E>(at) ^ at), dst + at);
-        }
-        if (with_v) {
-            const uint8_t* vs = vg + (size_t)(p0 >> 5) * SUB;
-#pragma unroll
-            for (int j = 0; j < NCP; ++j) {
-                const uint32_t at = (j * 4 + wv) * 256;
-                lds_dword(vs + at, (uint32_t)(lane * 4) ^ (v_swz<E>(at) ^ at), dst + SUB + at);
-            }
-        }
-    };
-    // Scores of the sub-block in stage st against the wave's 32 tokens.
-    auto score = [&](int st, v16f& acc) {
-        const uint8_t* kl = &ring[st][0][0];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-#pragma unroll
-        for (int m = 0; m < 16; ++m) {
-            v8bf16 kf;
-            if constexpr (KV8) {
-                const uint2 r = *(const uint2*)(kl + k_swz<1>((lane & 31) * 256 + (lane >> 5) * 128 + m * 8));
-                kf = kv_widen8(r.x, r.y, ksc);
-            } else {
-                kf = *(const v8bf16*)(kl + k_swz<2>((lane & 31) * 512 + (lane >> 5) * 256 + m * 16));
-            }
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[m], acc, 0, 0, 0);
-        }
-    };
-    const int t_max = min(t0 + 31, L - 1), t_top = min(T0 + 127, L - 1);  // the wave's and the workgroup's last token
-    const int nblocks = (S + L + 2047) / 2048;
-    for (int b = 0; b < nblocks; ++b) {
-        // Sub-blocks of 32 cache positions (aligned, as the transposed V cache is): the cached positions [c_lo, c_hi),
-        // then the positions [p_lo, p_hi) the chunk's own tokens o_lo .. o_hi - 1 were written to. n counts the
-        // workgroup's sub-blocks, nw this wave's (a prefix of them: the same positions in the same order).
-        const int c_lo = 2048 * b, c_hi = min(min(2048 * (b + 1), S), start);
-        const int o_lo = max(0, 2048 * b - S), o_end = min(2048 * (b + 1) - S, L);
-        const int o_hi = min(o_end, t_max + 1), o_top = min(o_end, t_top + 1);
-        const int p_lo = start + o_lo, p_hi = start + o_hi, p_al = p_lo & ~31;
-        const int n_c = c_hi > c_lo ? (c_hi - c_lo + 31) / 32 : 0;
-        const int n = n_c + (o_top > o_lo ? (start + o_top - p_al + 31) / 32 : 0);
-        const int nw = live ? n_c + (o_hi > o_lo ? (p_hi - p_al + 31) / 32 : 0) : 0;
-        if (n == 0) continue;
-        auto base = [&](int sb) { return sb < n_c ? c_lo + 32 * sb : p_al + 32 * (sb - n_c); };
-        // The rows r (positions base(sb) + r) of sub-block sb this lane's token sees: rlo <= r < rhi. Cached
-        // positions below c_hi; the chunk's from p_lo, below p_hi and up to the token's own.
-        auto window = [&](int sb, int& rlo, int& rhi) {
-            const int p0 = base(sb);
-            rlo = sb < n_c ? 0 : p_lo - p0;
-            rhi = (sb < n_c ? c_hi : min(p_hi, start + tq + 1)) - p0;
-        };
-        // Pass 1: the block's maximum per token.
-        float mx = -INFINITY;
-        copy(base(0), 0, false);
-        if (n > 1) copy(base(1), 1, false);
-        for (int sb = 0, st = 0; sb < n; ++sb, st = st == 2 ? 0 : st + 1) {
-            if (sb + 1 < n)
-                ring_ready<NCP>();
-            else
-                ring_ready<0>();
-            if (sb + 2 < n) copy(base(sb + 2), st == 0 ? 2 : st - 1, false);
-            v16f acc;
-            score(st, acc);
-            int rlo, rhi;
-            window(sb, rlo, rhi);
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int r = drow(i, lane);
-                mx = ((r >= rlo) & (r < rhi)) ? fmaxf(mx, rbf(acc[i])) : mx;
-            }
-        }
-        ring_release();
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float nb = fmaxf(best, mx);  // a token with nothing visible here keeps its maximum
-        const float scale = expf(best - nb);
-        // Pass 2: weights e^(s - max), their float32 sum, bf16 weights x V.
-        v16f pv[8];
-#pragma unroll
-        for (int db = 0; db < 8; ++db)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) pv[db][i] = 0.0f;
-        float wsum = 0.0f;
-        copy(base(0), 0, true);
-        if (n > 1) copy(base(1), 1, true);
-        for (int sb = 0, st = 0; sb < n; ++sb, st = st == 2 ? 0 : st + 1) {
-            if (sb + 1 < n)
-                ring_ready<2 * NCP>();
-            else
-                ring_ready<0>();
-            if (sb + 2 < n) copy(base(sb + 2), st == 0 ? 2 : st - 1, true);
-            {
-                v16f acc;
-                score(st, acc);
-                int rlo, rhi;
-                window(sb, rlo, rhi);
-                float w[16];
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int r = drow(i, lane);
-                    const float e = expf(rbf(acc[i]) - nb);
-                    w[i] = ((r >= rlo) & (r < rhi)) ? e : 0.0f;
-                }
-#pragma unroll
-                for (int i = 0; i < 16; ++i) wsum += w[i];
-                const uint8_t* vl = &ring[st][1][0];
-                typedef unsigned u4_ __attribute__((ext_vector_type(4)));
-#pragma unroll
-                for (int ks = 0; ks < 2; ++ks) {
-                    const u4_ pw = {pk_bf16(w[8 * ks + 0], w[8 * ks + 1]), pk_bf16(w[8 * ks + 2], w[8 * ks + 3]),
-                                    pk_bf16(w[8 * ks + 4], w[8 * ks + 5]), pk_bf16(w[8 * ks + 6], w[8 * ks + 7])};
-                    const v8bf16 pa = __builtin_bit_cast(v8bf16, pw);
-                    // Positions of this step in this lane: 16 ks + 4 (l / 32) + [0, 4) and 16 ks + 8 + 4 (l / 32) + [0, 4).
-                    const int q0 = 16 * ks + 4 * (lane >> 5);
-#pragma unroll
-                    for (int db = 0; db < 8; ++db) {
-                        const int d = db * 32 + (lane & 31);
-                        v8bf16 vw;
-                        if constexpr (KV8) {
-                            const uint32_t lo = *(const uint32_t*)(vl + v_swz<1>(d * 32 + q0));
-                            const uint32_t hi = *(const uint32_t*)(vl + v_swz<1>(d * 32 + q0 + 8));
-                            vw = kv_widen8(lo, hi, vsc);
-                        } else {
-                            const uint2 lo = *(const uint2*)(vl + v_swz<2>(d * 64 + q0 * 2));
-                            const uint2 hi = *(const uint2*)(vl + v_swz<2>(d * 64 + q0 * 2 + 16));
-                            vw = __builtin_bit_cast(v8bf16, (u4_){lo.x, lo.y, hi.x, hi.y});
-                        }
-                        pv[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa, vw, pv[db], 0, 0, 0);
-                    }
-                }
-            }
-        }
-        ring_release();
-        if (nw == 0) continue;  // nothing of this block is visible to the wave: it keeps its state
-        wsum += __shfl_xor(wsum, 32);
-        total = total * scale + wsum;
-        best = nb;
-        if (lane < 32) s_row[wv][lane] = scale;
-        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LDS writes land before its reads
-#pragma unroll
-        for (int db = 0; db < 8; ++db)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) so[db][i] = so[db][i] * s_row[wv][drow(i, lane)] + rbf(pv[db][i]);
+// Sub-blocks (of 32 aligned cache positions) a tile sees: the cached positions [0, start) in order, then its own
+// chunk's tokens 0 .. top, cut where the reference's blocks of [cache, chunk] end.
+struct PrefillSpan {
+    int S, start, n_c, first;  // first: own tokens before the first cut
+    __device__ __forceinline__ PrefillSpan(int S_, int start_)
+        : S(S_), start(start_), n_c((start_ + 31) >> 5), first(2048 - (S_ & 2047)) {}
+    __device__ __forceinline__ int own(int lo, int end) const {  // sub-blocks of own tokens [lo, end)
+        return end > lo ? ((start + end + 31) >> 5) - ((start + lo) >> 5) : 0;
     }
-    // out / total in bf16, times bf16 sigmoid(gate), e5m2 tiles for o_proj.
-    if (!live) return;
-    if (lane < 32) s_row[wv][lane] = total;
-    __builtin_amdgcn_s_waitcnt(0xc07f);
-    const int act_k = a.Hq * 256;
-#pragma unroll
-    for (int db = 0; db < 8; ++db)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int row = drow(i, lane), d = db * 32 + (lane & 31), t = t0 + row;
-            if (t >= L) continue;
-            const float o = rbf(so[db][i] / s_row[wv][row]);
-            const float gt = bf2f(a.qkv[(size_t)t * a.ld + (size_t)hq * 512 + 256 + d]);
-            a.act[act_offset(t, hq * 256 + d, act_k)] = (uint8_t)e5m2_byte(rbf(o * rbf(sigmoidf_(gt))));
-        }
+    __device__ __forceinline__ int count(int top) const {
+        int n = n_c;
+        for (int lo = 0, end = first; lo <= top; lo = end, end += 2048) n += own(lo, min(end, top + 1));
+        return n;
+    }
+};
+
+// One sub-block of a span: cache position p0, the positions [lo, hi) of it that belong to the span, whether they are
+// the chunk's own (then token t sees those up to start + t), and its block of the reference.
+struct PrefillSub {
+    int p0, lo, hi, own, block;
+};
+
+__device__ __forceinline__ PrefillSub prefill_sub(const PrefillSpan& sp, int top, int u) {
+    if (u < sp.n_c) return {u * 32, 0, sp.start, 0, u >> 6};
+    u -= sp.n_c;
+    int lo = 0, end = sp.first;
+    for (;; lo = end, end += 2048) {
+        const int n = sp.own(lo, min(end, top + 1));
+        if (u < n || end > top) break;
+        u -= n;
+    }
+    return {(((sp.start + lo) >> 5) + u) * 32, sp.start + lo, sp.start + min(end, top + 1), 1, (sp.S + lo) >> 11};
 }
 
-hipError_t q38_attn_prefill(const PrefillAttnArgs& a, hipStream_t stream) {
-    if (a.L < 1 || a.L % 32 || a.Hq % a.Hkv || a.S % 32) return hipErrorInvalidValue;
-    if (a.kv8) {
-        if (!a.k_scale || !a.v_scale) return hipErrorInvalidValue;
-        hipLaunchKernelGGL(attn_prefill_prep_kernel<true>, dim3(a.L), dim3(256), 0, stream, a);
-        if (!a.keys_only) hipLaunchKernelGGL(attn_prefill_kernel<true>, dim3(a.Hq, (a.L + 127) / 128), dim3(256), 0, stream, a);
-    } else {
-        hipLaunchKernelGGL(attn_prefill_prep_kernel<false>, dim3(a.L), dim3(256), 0, stream, a);
-        if (!a.keys_only) hipLaunchKernelGGL(attn_prefill_kernel<false>, dim3(a.Hq, (a.L + 127) / 128), dim3(256), 0, stream, a);
+// The item of this workgroup: tile (KV head, four wave tiles) and its range [u0, u1) of sub-blocks. Ranges per tile: the
+// count up to ns_max that ends the last tile first when every CU takes items of 1 / count of the longest tile, each with
+// a fixed cost of about six sub-blocks (queries, first loads, output). Workgroups start in id order and go to the XCDs in turn:
+// ranges outermost, so that an XCD's workgroups stream the same part of one KV head (8 / Hkv XCDs per head) through its
+// L2; the tiles with the latest tokens, the longest, first.
+struct PrefillItem {
+    int kvh, quad, top, u0, u1, ns, z;
+};
+
+__device__ __forceinline__ bool prefill_item(const PrefillAttnArgs& a, const PrefillSpan& sp, int id, PrefillItem& it) {
+    const int G = a.Hq / a.Hkv, ntt = (a.L + PF_ROWS - 1) / PF_ROWS, nq = (G * ntt + 3) / 4;
+    const int longest = sp.count(a.L - 1), tiles = nq * a.Hkv;
+    int ns = 1, best = 0x7fffffff;
+    for (int c = 1; c <= a.ns_max && (c == 1 || longest >= 4 * c); ++c) {
+        const int cost = ((tiles * c + a.cus - 1) / a.cus) * ((longest + c - 1) / c + 6);
+        if (cost < best) best = cost, ns = c;
     }
+    int j;
+    if (a.Hkv <= 8 && 8 % a.Hkv == 0) {
+        const int per = 8 / a.Hkv, x = id & 7;
+        it.kvh = x / per;
+        j = (id >> 3) * per + x % per;
+    } else {
+        it.kvh = id % a.Hkv;
+        j = id / a.Hkv;
+    }
+    if (j >= nq * ns) return false;
+    it.ns = ns;
+    it.z = j / nq;
+    it.quad = nq - 1 - j % nq;
+    const int last = min(it.quad * 4 + 3, G * ntt - 1);  // the quad's last tile with tokens
+    it.top = min((last / G) * PF_ROWS + PF_ROWS - 1, a.L - 1);
+    const int n = sp.count(it.top);
+    it.u0 = (int)((long)it.z * n / ns);
+    it.u1 = (int)((long)(it.z + 1) * n / ns);
+    return true;
+}
+
+// Partial slots: (KV head, quad, range), of 4 waves x 64 tokens x 256 dims floats, and 2 floats per token.
+__device__ __forceinline__ size_t prefill_slot(const PrefillAttnArgs& a, int kvh, int quad, int z) {
+    const int nq = (a.Hq / a.Hkv * ((a.L + PF_ROWS - 1) / PF_ROWS) + 3) / 4;
+    return (size_t)(kvh * nq + quad) * a.ns_max + z;
+}
+
+__device__ __forceinline__ float order_float(int i) { return __int_as_float(i >= 0 ? i : i ^ 0x7fffffff); }
+
+// 16 bytes per lane from base + off (base wave-uniform) to LDS dst + 16 l (dst wave-uniform), as lds_dword.
+__device__ __forceinline__ void lds_quad(const void* base, uint32_t off, uint32_t dst) {
+    const uint32_t m0 = __builtin_amdgcn_readfirstlane(dst);
+    asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(m0) : "memory");
+}
+
+__device__ __forceinline__ v8bf16 lds_frag(uint32_t at) {
+    return *(const __attribute__((address_space(3))) v8bf16*)(uintptr_t)at;
+}
+
+// A sub-block in LDS and how the MFMAs read it.
+// K: row r holds cache position p0 + pi(r), pi swapping bits 2 and 3: with the keys as A and the queries as B, lane l
+//    (token l % 32, half h = l / 32) then holds the scores of positions 16 (i / 8) + 8 h + i % 8, the eight consecutive
+//    positions that MFMA step i / 8 of weights x V takes from a lane, so scores become operands without moving. Row r's
+//    16-byte chunk c sits at c ^ (r % 16), which spreads a read of 32 rows over the banks.
+// V: row d (dim) of 32 positions, its 16-byte chunk c at c ^ f(d), f(d) = (d / 2) % 4 ^ (d / 8) % 2.
+struct SubCopy {
+    const uint8_t *kg, *vg;
+    uint32_t lane_k, lane_v, lds0;
+    int wv;
+    __device__ __forceinline__ void init(const bf16_t* k, const bf16_t* v, size_t head, int S, int lane, int wv_, uint32_t lds) {
+        kg = (const uint8_t*)(k + head * S * 256);
+        vg = (const uint8_t*)(v + head * S * 256);
+        wv = wv_;
+        lds0 = lds;
+        lane_k = (lane >> 5) * 512 + (((lane & 31) ^ (2 * wv + (lane >> 5))) << 4);
+        const int d = lane >> 2;
+        lane_v = d * 64 + (((lane & 3) ^ (((d >> 1) & 3) ^ ((d >> 3) & 1))) << 4);
+    }
+    __device__ __forceinline__ void keys(int p0, uint32_t at) const {
+        const uint8_t* src = kg + (size_t)p0 * 512;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int r = 8 * j + 2 * wv, q = (r & ~12) | (r & 4) << 1 | (r & 8) >> 1;  // pi(r)
+            lds_quad(src + q * 512, j & 1 ? lane_k ^ 128 : lane_k, at + r * 512);
+        }
+    }
+    __device__ __forceinline__ void values(int p0, uint32_t at) const {
+        const uint8_t* src = vg + (size_t)(p0 >> 5) * PF_SUB;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) lds_quad(src + (j * 4 + wv) * 1024, lane_v, at + (j * 4 + wv) * 1024);
+    }
+};
+
+// The wave's tile: query head and first token, and its queries in registers (zero past the chunk).
+struct PrefillTile {
+    int hq, t0;
+    bool live;
+};
+
+__device__ __forceinline__ PrefillTile prefill_tile(const PrefillAttnArgs& a, int kvh, int id) {
+    const int G = a.Hq / a.Hkv, t0 = (id / G) * PF_ROWS;
+    return {kvh * G + id % G, t0, t0 < a.L};
+}
+
+__device__ __forceinline__ void prefill_queries(const PrefillAttnArgs& a, const PrefillTile& tl, int lane, v8bf16 (&qf)[2][16]) {
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+        const int t = min(tl.t0 + rt * 32, a.L - 32);  // past the chunk (L is a multiple of 32): its last tokens, never used
+        const bf16_t* qp = a.qs + ((size_t)tl.hq * a.L + t + (lane & 31)) * QP + (lane >> 5) * 128;
+#pragma unroll
+        for (int m = 0; m < 16; ++m) qf[rt][m] = load8p(qp + m * 8);
+    }
+}
+
+// Scores of the sub-block whose keys are at LDS address kl (this lane's row), operands read four MFMA pairs ahead. The
+// fences hold that order: left alone, the compiler gathers all sixteen reads first, and spills.
+__device__ __forceinline__ void prefill_scores(uint32_t kl, const v8bf16 (&qf)[2][16], v16f (&s)[2]) {
+    v16f zero;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) zero[i] = 0.0f;
+    v8bf16 kf[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) kf[m] = lds_frag(kl ^ (m << 4));
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+        __builtin_amdgcn_sched_barrier(0);
+        s[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[m & 3], qf[0][m], m ? s[0] : zero, 0, 0, 0);
+        s[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[m & 3], qf[1][m], m ? s[1] : zero, 0, 0, 0);
+        if (m < 12) kf[m & 3] = lds_frag(kl ^ ((m + 4) << 4));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// Scores of positions a lane's token does not see become -inf (weight zero): those outside [lo, hi), and of the
+// chunk's own those after the token. Only sub-blocks at an edge need it.
+__device__ __forceinline__ bool prefill_whole(const PrefillSub& sb, const PrefillTile& tl, int start) {
+    return sb.p0 >= sb.lo && sb.p0 + 32 <= sb.hi && (!sb.own || sb.p0 + 31 <= start + tl.t0);
+}
+__device__ __forceinline__ void prefill_mask(const PrefillSub& sb, const PrefillTile& tl, int start, int lane, v16f (&s)[2]) {
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+        const int t = tl.t0 + rt * 32 + (lane & 31), h8 = (lane >> 5) * 8;
+        const int hi = sb.own ? min(sb.hi, start + t + 1) : sb.hi;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int p = sb.p0 + 16 * (i >> 3) + h8 + (i & 7);
+            if (p < sb.lo || p >= hi) s[rt][i] = -INFINITY;
+        }
+    }
+}
+
+}  // namespace
+
+// Largest score of each token over each block of the reference, into mx [Hq][blocks][L] (ordered ints, reset by the
+// prep kernel) by integer maxima, which do not depend on the order.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill_max_kernel(const PrefillAttnArgs a) {
+    __shared__ __attribute__((aligned(1024))) uint8_t ring[4][PF_SUB];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int slot = *a.slot, start = *a.start;
+    if (start < 0 || start + a.L > a.S || slot < 0 || slot >= a.rows) return;  // the host checks these too
+    const PrefillSpan sp(a.S, start);
+    PrefillItem it;
+    if (!prefill_item(a, sp, blockIdx.x, it)) return;
+    const int n = it.u1 - it.u0;
+    if (n <= 0) return;
+    const PrefillTile tl = prefill_tile(a, it.kvh, it.quad * 4 + wv);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)LDS_PTR(&ring[0][0]);
+    SubCopy cp;
+    cp.init(a.kw, a.vw, (size_t)(a.kw_slot ? slot : 0) * a.Hkv + it.kvh, a.S, lane, wv, lds0);
+    v8bf16 qf[2][16];
+    prefill_queries(a, tl, lane, qf);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+        if (i < n) cp.keys(prefill_sub(sp, it.top, it.u0 + i).p0, lds0 + i * PF_SUB);
+    const uint32_t kl = (lane & 31) * 512 + (lane >> 5) * 256 + ((lane & 15) << 4);
+    float mx[2] = {-INFINITY, -INFINITY};
+    const int nblk = (a.S + a.L + 2047) >> 11;
+    auto flush = [&](int block) {
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) {
+            // The largest bf16 score is the largest score in bf16.
+            const float m = rbf(fmaxf(mx[rt], __shfl_xor(mx[rt], 32)));
+            const int t = tl.t0 + rt * 32 + (lane & 31);
+            if (lane < 32 && tl.live && t < a.L && m > -INFINITY) atomicMax(a.mx + ((size_t)tl.hq * nblk + block) * a.L + t, order_bits(m));
+            mx[rt] = -INFINITY;
+        }
+    };
+    PrefillSub sb = prefill_sub(sp, it.top, it.u0);
+    for (int i = 0; i < n; ++i) {
+        if (i + 2 < n)
+            ring_ready<8>();
+        else
+            ring_ready<0>();
+        if (i + 3 < n) cp.keys(prefill_sub(sp, it.top, it.u0 + i + 3).p0, lds0 + ((i + 3) & 3) * PF_SUB);
+        v16f s[2];
+        prefill_scores(lds0 + (i & 3) * PF_SUB + kl, qf, s);
+        if (!prefill_whole(sb, tl, start)) prefill_mask(sb, tl, start, lane, s);
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) mx[rt] = fmaxf(mx[rt], s[rt][e]);
+        const int block = sb.block;
+        if (i + 1 < n) sb = prefill_sub(sp, it.top, it.u0 + i + 1);
+        if (i + 1 == n || sb.block != block) flush(block);
+    }
+}
+
+// Weights x V of one item: per sub-block the scores again, the weights e^(s - m) with m the running maximum through the
+// sub-block's block, their float32 sums, and the bf16 weights times V; at a block's end the sums so far are rescaled
+// to the next block's maximum. V as A and the weights as B, so that a lane holds four consecutive dims of one token
+// (the order the activation tiles and the float4 partials want) and its row factors are its own. Sub-block i's
+// weights x V run beside sub-block i + 1's scores, whose weights are formed beside them (the loop body has no branch
+// but the edges), with the copies two sub-blocks ahead.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void attn_prefill_kernel(const PrefillAttnArgs a) {
+    __shared__ __attribute__((aligned(1024))) uint8_t ring[4][2][PF_SUB];  // [stage][K, V]
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int slot = *a.slot, start = *a.start;
+    if (start < 0 || start + a.L > a.S || slot < 0 || slot >= a.rows) return;
+    const PrefillSpan sp(a.S, start);
+    PrefillItem it;
+    if (!prefill_item(a, sp, blockIdx.x, it)) return;
+    const int n = it.u1 - it.u0;
+    const PrefillTile tl = prefill_tile(a, it.kvh, it.quad * 4 + wv);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)LDS_PTR(&ring[0][0][0]);
+    SubCopy cp;
+    cp.init(a.kw, a.vw, (size_t)(a.kw_slot ? slot : 0) * a.Hkv + it.kvh, a.S, lane, wv, lds0);
+    v8bf16 qf[2][16];
+    prefill_queries(a, tl, lane, qf);
+    auto copy = [&](int i) {
+        const int p0 = prefill_sub(sp, it.top, it.u0 + i).p0;
+        const uint32_t at = lds0 + (i & 3) * 2 * PF_SUB;
+        cp.keys(p0, at);
+        cp.values(p0, at + PF_SUB);
+    };
+    for (int i = 0; i < min(n, 2); ++i) copy(i);
+    const uint32_t kl = (lane & 31) * 512 + (lane >> 5) * 256 + ((lane & 15) << 4);
+    const int fd = ((lane >> 1) & 3) ^ ((lane >> 3) & 1);
+    const uint32_t vl = PF_SUB + (lane & 31) * 64 + (((lane >> 5) ^ fd) << 4);
+
+    const int nblk = (a.S + a.L + 2047) >> 11;
+    float nb[2] = {2.0f * -1e4f, 2.0f * -1e4f}, total[2] = {0.0f, 0.0f};
+    int known = -1;  // blocks whose maxima nb holds
+    auto raise = [&](int block) {
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) {
+            const int* mp = a.mx + (size_t)tl.hq * nblk * a.L + min(tl.t0 + rt * 32, a.L - 32) + (lane & 31);
+            if (tl.live)
+                for (int b = known + 1; b <= block; ++b) nb[rt] = fmaxf(nb[rt], order_float(mp[(size_t)b * a.L]));
+        }
+        known = block;
+    };
+    v16f o[2][8];  // o[rt][db][e]: token 32 rt + l % 32, dim 32 db + 8 (e / 4) + 4 (l / 32) + e % 4
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int db = 0; db < 8; ++db)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) o[rt][db][e] = 0.0f;
+    v16f s[2];
+    // Two of the sub-block's weights (x: token tile x / 8, MFMA step x / 4 % 2, word x % 4) into w.
+    typedef uint32_t u4_ __attribute__((ext_vector_type(4)));
+    auto weight2 = [&](int x, u4_ (&w)[2][2]) __attribute__((always_inline)) {
+        const int rt = x >> 3, e = 2 * (x & 7);
+        const uint32_t r = pk_bf16(s[rt][e], s[rt][e + 1]);
+        const float e0 = __builtin_amdgcn_exp2f((lo_bf(r) - nb[rt]) * LOG2E);
+        const float e1 = __builtin_amdgcn_exp2f((hi_bf(r) - nb[rt]) * LOG2E);
+        total[rt] += e0;
+        total[rt] += e1;
+        w[rt][(x >> 2) & 1][x & 3] = pk_bf16(e0, e1);
+    };
+    u4_ pw[2][2];  // [token tile][MFMA step]: the sub-block's bf16 weights
+    // Weights x V of sub-block i (MFMA step x: dims 32 (x / 2), positions 16 (x % 2) + [0, 16)), with the next
+    // sub-block's weights formed beside the MFMAs.
+    auto values = [&](int i, auto next) __attribute__((always_inline)) {
+        const uint32_t va = lds0 + (i & 3) * 2 * PF_SUB + vl;
+        auto frag = [&](int x) __attribute__((always_inline)) { return lds_frag((va ^ ((x & 1) << 5)) + (x >> 1) * 2048); };
+        v8bf16 vf[4];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) vf[x] = frag(x);
+        u4_ nw[2][2];
+#pragma unroll
+        for (int x = 0; x < 16; ++x) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int rt = 0; rt < 2; ++rt)
+                o[rt][x >> 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[x & 3], __builtin_bit_cast(v8bf16, pw[rt][x & 1]),
+                                                                       o[rt][x >> 1], 0, 0, 0);
+            if (x < 12) vf[x & 3] = frag(x + 4);
+            if constexpr (decltype(next)::value) weight2(x, nw);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (decltype(next)::value) {
+#pragma unroll
+            for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) pw[rt][ks] = nw[rt][ks];
+        }
+    };
+    // Sub-block i landed (and every wave past sub-block i - 2's operands), sub-block i + 2's copies issued, i's scores.
+    auto scores = [&](int i) __attribute__((always_inline)) {
+        if (i + 1 < n)
+            ring_ready<8>();
+        else
+            ring_ready<0>();
+        if (i + 2 < n) copy(i + 2);
+        prefill_scores(lds0 + (i & 3) * 2 * PF_SUB + kl, qf, s);
+        asm volatile("" : "+v"(s[0]), "+v"(s[1]));  // in VGPRs, where the weights are formed; the AGPRs hold o
+        const PrefillSub sb = prefill_sub(sp, it.top, it.u0 + i);
+        if (!prefill_whole(sb, tl, start)) prefill_mask(sb, tl, start, lane, s);
+    };
+    // One block of the reference at a time: between them the sums are rescaled, so the inner loop only accumulates.
+    for (int i = 0; i < n;) {
+        const int block = prefill_sub(sp, it.top, it.u0 + i).block;
+        int end = i + 1;  // this block's sub-blocks end here
+        if (it.u0 + i < sp.n_c) end = min(n, min(sp.n_c, (it.u0 + i | 63) + 1) - it.u0);
+        while (end < n && prefill_sub(sp, it.top, it.u0 + end).block == block) ++end;
+        const float b0 = nb[0], b1 = nb[1];
+        raise(block);
+        if (i > 0) {
+            const float f[2] = {__builtin_amdgcn_exp2f((b0 - nb[0]) * LOG2E), __builtin_amdgcn_exp2f((b1 - nb[1]) * LOG2E)};
+#pragma unroll
+            for (int rt = 0; rt < 2; ++rt) {
+                total[rt] *= f[rt];
+#pragma unroll
+                for (int db = 0; db < 8; ++db)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) o[rt][db][e] *= f[rt];
+            }
+        }
+        scores(i);
+#pragma unroll
+        for (int x = 0; x < 16; ++x) weight2(x, pw);
+        for (; i < end - 1; ++i) {
+            scores(i + 1);
+            values(i, std::true_type{});
+        }
+        values(i++, std::false_type{});
+    }
+    if (!tl.live) return;
+    // The range's sums, [wave][rt][db][e / 4][lane] float4, and per token its maximum and weight sum.
+    const size_t sl = prefill_slot(a, it.kvh, it.quad, it.z);
+    float* po = a.part + sl * (4 * PF_ROWS * 256) + (size_t)wv * (PF_ROWS * 256) + lane * 4;
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+#pragma unroll
+        for (int db = 0; db < 8; ++db)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *(v4f*)(po + ((rt * 8 + db) * 4 + q) * 256) =
+                    (v4f){o[rt][db][4 * q], o[rt][db][4 * q + 1], o[rt][db][4 * q + 2], o[rt][db][4 * q + 3]};
+        const float sum = total[rt] + __shfl_xor(total[rt], 32);
+        if (lane < 32) *(float2*)(a.part_rows + (sl * 4 * PF_ROWS + wv * PF_ROWS + rt * 32 + lane) * 2) = make_float2(nb[rt], sum);
+    }
+}
+
+// The ranges of one wave tile added in order, out / total in bf16, times bf16 sigmoid(gate), e5m2 tiles for o_proj. Grid
+// (wave tiles of 64 tokens x 4): wave w of block q takes 32 tokens and 64 dims, a lane 4 dims of one token at a time. The
+// reference rounds each block's weights x V to bf16; with all of a token's positions in one block that rounding is the
+// sum's, and kept, and over several blocks the float32 sums are used as they are.
+__global__ __launch_bounds__(256) void attn_prefill_finish_kernel(const PrefillAttnArgs a) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int slot = *a.slot, start = *a.start;
+    if (start < 0 || start + a.L > a.S || slot < 0 || slot >= a.rows) return;
+    const PrefillSpan sp(a.S, start);
+    const int G = a.Hq / a.Hkv, ntt = (a.L + PF_ROWS - 1) / PF_ROWS;
+    const int kvh = blockIdx.y, tile = blockIdx.x >> 2, quad = tile >> 2, w = tile & 3;
+    PrefillItem it;
+    if (tile >= G * ntt || !prefill_item(a, sp, 0, it)) return;
+    const PrefillTile tl = prefill_tile(a, kvh, tile);
+    const int rt = wv & 1, db0 = ((blockIdx.x & 3) * 2 + (wv >> 1)), t = tl.t0 + rt * 32 + (lane & 31);
+    if (tl.t0 + rt * 32 >= a.L) return;
+    const size_t sl = prefill_slot(a, kvh, quad, 0);
+    const float* rows = a.part_rows + (sl * 4 * PF_ROWS + w * PF_ROWS + rt * 32 + (lane & 31)) * 2;
+    const float M = rows[(size_t)(it.ns - 1) * 4 * PF_ROWS * 2];  // the last range's maximum is the largest
+    const bool one = (start == 0 || start <= 2048) && (a.S + t) >> 11 == (start > 0 ? 0 : a.S >> 11);
+    float total = 0.0f;
+    v4f o[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) o[q] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+    for (int z = 0; z < it.ns; ++z) {
+        const float2 r = *(const float2*)(rows + (size_t)z * 4 * PF_ROWS * 2);
+        const float f = __builtin_amdgcn_exp2f((r.x - M) * LOG2E);
+        total += r.y * f;
+        const float* po = a.part + (sl + z) * (4 * PF_ROWS * 256) + (size_t)w * (PF_ROWS * 256) + (rt * 8 + db0) * 1024 + lane * 4;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const v4f v = *(const v4f*)(po + q * 256);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[q][e] += v[e] * f;
+        }
+    }
+    const int act_k = a.Hq * 256;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int d = db0 * 32 + q * 8 + (lane >> 5) * 4;
+        const uint2 g = *(const uint2*)(a.qkv + (size_t)t * a.ld + (size_t)tl.hq * 512 + 256 + d);
+        const float gt[4] = {lo_bf(g.x), hi_bf(g.x), lo_bf(g.y), hi_bf(g.y)};
+        float r[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float v = rbf((one ? rbf(o[q][e]) : o[q][e]) / total);
+            r[e] = rbf(v * rbf(sigmoidf_(gt[e])));
+        }
+        *(uint32_t*)(a.act + act_offset(t, tl.hq * 256 + d, act_k)) = pk_e5m2(r[0], r[1], r[2], r[3]);
+    }
+}
+
+// An FP8 cache's row `slot` as bf16(e4m3 x scale), positions up to the chunk's end: the operands attn_prefill_max and
+// attn_prefill read, widened once instead of by every tile. Grid (32 positions, KV head).
+__global__ __launch_bounds__(256) void attn_prefill_widen_kernel(const PrefillAttnArgs a) {
+    const int slot = *a.slot, start = *a.start, p0 = blockIdx.x * 32;
+    if (start < 0 || start + a.L > a.S || slot < 0 || slot >= a.rows || p0 >= start + a.L) return;
+    const size_t src = ((size_t)slot * a.Hkv + blockIdx.y) * a.S * 256 + (size_t)p0 * 256;
+    const size_t dst = (size_t)blockIdx.y * a.S * 256 + (size_t)p0 * 256;
+    const float ksc = bf2f(*a.k_scale), vsc = bf2f(*a.v_scale);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const size_t e = (size_t)(i * 256 + threadIdx.x) * 8;
+        const uint2 k = *(const uint2*)((const uint8_t*)a.k_cache + src + e), v = *(const uint2*)((const uint8_t*)a.v_cache + src + e);
+        *(v8bf16*)(a.k_wide + dst + e) = kv_widen8(k.x, k.y, ksc);
+        *(v8bf16*)(a.v_wide + dst + e) = kv_widen8(v.x, v.y, vsc);
+    }
+}
+
+hipError_t q38_attn_prefill(const PrefillAttnArgs& a0, hipStream_t stream) {
+    PrefillAttnArgs a = a0;
+    if (a.L < 1 || a.L % 32 || a.Hq % a.Hkv || a.S % 32) return hipErrorInvalidValue;
+    if (a.kv8 && (!a.k_scale || !a.v_scale)) return hipErrorInvalidValue;
+    if (a.kv8)
+        hipLaunchKernelGGL(attn_prefill_prep_kernel<true>, dim3(a.L), dim3(256), 0, stream, a);
+    else
+        hipLaunchKernelGGL(attn_prefill_prep_kernel<false>, dim3(a.L), dim3(256), 0, stream, a);
+    if (a.keys_only) return hipGetLastError();
+    const int tiles = (a.Hq / a.Hkv) * ((a.L + PF_ROWS - 1) / PF_ROWS), quads = (tiles + 3) / 4 * a.Hkv;
+    a.ns_max = std::min(PREFILL_RANGES, std::max(1, PREFILL_ITEMS / quads));
+    a.cus = q38_device_cus();
+    if ((size_t)quads * a.ns_max > a.part_slots) return hipErrorInvalidValue;
+    a.kw = a.k_cache;
+    a.vw = a.v_cache;
+    a.kw_slot = 1;
+    if (a.kv8) {
+        hipLaunchKernelGGL(attn_prefill_widen_kernel, dim3(a.S / 32, a.Hkv), dim3(256), 0, stream, a);
+        a.kw = a.k_wide;
+        a.vw = a.v_wide;
+        a.kw_slot = 0;
+    }
+    // Every item has an id: with 8 / Hkv XCDs per KV head the ids come in rounds of eight, one item per XCD.
+    const int per_head = (tiles + 3) / 4 * a.ns_max;
+    const int grid = a.Hkv <= 8 && 8 % a.Hkv == 0 ? (per_head + 8 / a.Hkv - 1) / (8 / a.Hkv) * 8 : per_head * a.Hkv;
+    hipLaunchKernelGGL(attn_prefill_max_kernel, dim3(grid), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(attn_prefill_kernel, dim3(grid), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(attn_prefill_finish_kernel, dim3(tiles * 4, a.Hkv), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 
