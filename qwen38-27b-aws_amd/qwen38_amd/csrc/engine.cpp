@@ -93,7 +93,7 @@ struct q38_handle {
         off_sp_sin, off_sp_states, off_sp_out, off_sp_current, off_sp_ids, off_sp_at, off_sp_draft, off_gemm, off_gates, off_status,
         workspace_bytes;
     // prefill scratch (with a prefill chunk in the config)
-    size_t off_pqn = 0, off_pkn = 0, off_pv = 0, off_po = 0, off_pbeta = 0, off_pg = 0, off_pqs = 0, off_pmx = 0, off_ppart = 0,
+    size_t off_pqn = 0, off_pkn = 0, off_pv = 0, off_po = 0, off_pdecay = 0, off_ppt = 0, off_pqs = 0, off_pmx = 0, off_ppart = 0,
            off_prows = 0, off_pkw = 0, off_pvw = 0;
     size_t part_floats;  // capacity of the split-K partial buffer
     int gate_groups;  // K ranges of the gated-delta gate projections
@@ -409,10 +409,10 @@ int run_mixer(q38_handle* h, int li, const StepIO& io, int rd, int wr, hipStream
             p.conv = conv + (size_t)rd * h->B * h->C * 3;  // the current half, in place
             p.qn = (float*)h->ws(h->off_pqn);
             p.kn = (float*)h->ws(h->off_pkn);
-            p.v = (float*)h->ws(h->off_pv);
-            p.beta = (float*)h->ws(h->off_pbeta);
-            p.g = (float*)h->ws(h->off_pg);
-            p.o = (float*)h->ws(h->off_po);
+            p.v = (bf16_t*)h->ws(h->off_pv);
+            p.decay = (float*)h->ws(h->off_pdecay);
+            p.pt = (float*)h->ws(h->off_ppt);
+            p.o = (bf16_t*)h->ws(h->off_po);
             p.act = act_mid;
             p.eps = h->cfg.rms_norm_eps;
             HIP_TRY(q38_gdn_prefill(p, stream));
@@ -741,10 +741,10 @@ int q38_create(const q38_config* cfg, q38_handle** out) {
     if (Tc) {
         h->off_pqn = take(Tc * h->Hk * h->dk * 4);
         h->off_pkn = take(Tc * h->Hk * h->dk * 4);
-        h->off_pv = take(Tc * h->Hv * h->dk * 4);
-        h->off_po = take(Tc * h->Hv * h->dk * 4);
-        h->off_pbeta = take(Tc * h->Hv * 4);
-        h->off_pg = take(Tc * h->Hv * 4);
+        h->off_pv = take(Tc * h->Hv * h->dk * 2);
+        h->off_po = take(Tc * h->Hv * h->dk * 2);
+        h->off_ppt = take(Tc / PREFILL_GDN_CHUNK * h->Hv * 2 * PREFILL_GDN_CHUNK * PREFILL_GDN_CHUNK * 4);
+        h->off_pdecay = take(Tc * h->Hv * 3 * 4);
         h->off_pqs = take((size_t)h->Hq * Tc * 256 * 2);
         h->off_pmx = take((size_t)h->Hq * ((h->S + Tc + 2047) / 2048) * Tc * 4);
         h->prefill_slots = prefill_slots(c.prefill_chunk, h->Hq, h->Hkv);

@@ -86,6 +86,8 @@ struct GdnArgs {
     bf16_t* out_probe;       // optional [B*K][Hv*128]: the in-step output o (bf16) before the gated norm
 };
 
+constexpr int PREFILL_GDN_CHUNK = 32;  // tokens the delta rule takes at a time (prefill calls hold a multiple of 32)
+
 // Gated delta net over one prefill chunk of one row (prefill.hip).
 struct PrefillGdnArgs {
     int L, Hk, Hv, C;
@@ -105,10 +107,11 @@ struct PrefillGdnArgs {
     bf16_t* conv;            // [B][C][3], the current half: row slot read and replaced
     float* qn;               // scratch [L][Hk][128]: normed q times d^-1/2
     float* kn;               // scratch [L][Hk][128]
-    float* v;                // scratch [L][Hv][128]
-    float* beta;             // scratch [L][Hv]
-    float* g;                // scratch [L][Hv]
-    float* o;                // scratch [L][Hv][128]
+    bf16_t* v;               // scratch [L][Hv][128]
+    float* decay;            // scratch [L / chunk][Hv][3][chunk]: beta, e^c and e^(c_last - c), c the log decays summed from
+                             // the chunk's first token on
+    float* pt;               // scratch [L / chunk][Hv][T, P][chunk][chunk], chunk = PREFILL_GDN_CHUNK
+    bf16_t* o;               // scratch [L][Hv][128]
     uint8_t* act;            // e5m2 activation tiles of width Hv*128 for out_proj
     float eps;
 };

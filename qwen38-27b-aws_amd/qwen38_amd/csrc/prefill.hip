@@ -3,14 +3,13 @@
 // attention, 843-855 for the MTP layer's cache-only form).
 //
 // Gated delta net, after the qkvz GEMM and the gates kernel over the chunk:
-//   gdn_prefill_prep   (token, key head): conv over the chunk with the row's conv history (bf16 tap products summed
-//                      by bf16 additions, model.py:514), SiLU, l2 norms of q and k, the gates times `valid`
-//   gdn_prefill_scan   (value head, 32 state columns): the gated delta rule token by token in float32 from the row's
-//                      state (times `start > 0`), the state kept in registers, the tokens' k, q, v, beta and g staged
-//                      through LDS a round ahead; per token S = e^g S, delta = (v - S^T
-//                      k) beta, S += k delta^T, o = S^T q. The reference runs the same rule in pieces of 128 tokens
-//                      (chunked_gated_delta, model.py:88-124); both are the same sums in float32, in another order.
-//   gdn_prefill_finish (token, 4 value heads): o to bf16, gated RMS norm times SiLU(z), e5m2 tiles for out_proj
+//   gdn_prefill_prep   (32 tokens, key head): conv over the chunk with the row's conv history (bf16 tap products summed
+//                      by bf16 additions, model.py:514), SiLU, l2 norms of q and k, the gates times `valid`; the
+//                      state-independent matrices of the delta rule over these tokens
+//   gdn_prefill_scan   (value head, 32 state columns): the gated delta rule (per token S = e^g S, delta = (v - S^T k)
+//                      beta, S += k delta^T, o = S^T q) in chunks of 32 tokens from the row's state (times `start > 0`), in
+//                      float32 on the matrix cores
+//   gdn_prefill_finish (4 tokens, 4 value heads): gated RMS norm of bf16 o times SiLU(z), e5m2 tiles for out_proj
 //   gdn_prefill_carry  the row's new conv state: the three inputs from n_valid on of [history, chunk]
 //
 // Attention, after the qkv GEMM over the chunk:
@@ -31,168 +30,398 @@
 
 namespace {
 
+constexpr int GC = PREFILL_GDN_CHUNK;  // tokens of one chunk of the delta rule
+
 __device__ __forceinline__ float conv_window(const PrefillGdnArgs& a, const bf16_t* hist, float keep, int c, int w) {
     // Input w of channel c's window: the row's conv history (times keep) for w < 3, then the chunk's inputs.
     return w < 3 ? bf2f(hist[(size_t)c * 3 + w]) * keep : bf2f(a.qkv[(size_t)(w - 3) * a.C + c]);
 }
 
+__device__ __forceinline__ v4f mfma16(float x, float y, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0); }
+
+// Direct global -> LDS copy of 16 bytes per lane from base + off (base wave-uniform, in scalar registers): lane l's bytes
+// land at LDS address dst + 16 l (dst wave-uniform). Inline assembly, so the compiler neither counts it nor waits for it;
+// the kernels' own vmcnt waits cover it.
+__device__ __forceinline__ void lds_quad(const void* base, uint32_t off, uint32_t dst) {
+    const uint32_t m0 = __builtin_amdgcn_readfirstlane(dst);
+    asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(m0) : "memory");
+}
+
+// e^x of a 64-bit x, in float32 without x's own rounding (|x| ulps of the result).
+__device__ __forceinline__ float exp_of(double x) {
+    const float hi = (float)x, e = expf(hi);
+    return e + e * (float)(x - hi);
+}
+
+// This wave's LDS accesses are done; then meet the other waves (loads from global memory stay in flight).
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 }  // namespace
 
+// Grid (32 tokens, key head): conv, SiLU, l2 norms and gates of the tokens, then what a chunk of the delta rule needs that
+// does not depend on the state. With c_t the log decays summed from the chunk's start, k . k and q . k on the float32 MFMA, and per
+// value head M_ts = beta_t e^(c_t - c_s) k_t . k_s (s < t), T = (I + M)^-1 by forward substitution (a column per lane),
+// P_ts = e^(c_t - c_s) q_t . k_s (s <= t).
+// Bounds: the conv's and SiLU's arithmetic (about 40 instructions per input at a bf16 rounding after each operation; the
+// memory traffic, 145 MB for 2,048 tokens of the 27B layer, is half its time). Wave w takes tokens 8 w .. 8 w + 7 of one
+// head after another, a lane two channels, each input loaded once for the four taps, the next head's meanwhile: 60 us
+// with the matrices, where one token and channel per thread took 152 us for the conv and norms alone.
 __global__ __launch_bounds__(256) void gdn_prefill_prep_kernel(const PrefillGdnArgs a) {
-    constexpr int D = 128, GMAX = 8;
-    __shared__ float red[4];
-    const int t = blockIdx.x, kh = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int D = 128, GMAX = 8, KP = D + 4, MP = GC + 4;
+    __shared__ __attribute__((aligned(16))) float sk[GC][KP], sq[GC][KP], sm[4][GC][MP];
+    __shared__ float sb[4][GC];
+    __shared__ double sc[4][GC];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ch = blockIdx.x, t0 = ch * GC, kh = blockIdx.y;
     const int Hk = a.Hk, Hv = a.Hv, C = a.C, rep = Hv / Hk;
-    const int slot = *a.slot;
+    const int slot = *a.slot, nv = *a.n_valid;
     if (slot < 0 || slot >= a.rows) return;
-    const float keep = *a.start > 0 ? 1.0f : 0.0f, valid = t < *a.n_valid ? 1.0f : 0.0f;
+    const float keep = *a.start > 0 ? 1.0f : 0.0f;
     const bf16_t* hist = a.conv + (size_t)slot * C * 3;
 
-    // Gates of this key head's value heads (model.py:333-337, 499-500).
-    if (tid < 2 * rep) {
-        const int h = kh * rep + tid % rep, which = tid / rep, O = 2 * Hv;
-        const float* p = a.gate_part + (size_t)t * O + (which ? Hv + h : h);
-        float sum = 0.0f;
-#pragma unroll
-        for (int gi = 0; gi < GMAX; ++gi)
-            if (gi < a.gate_groups) sum += p[(size_t)gi * a.L * O];
-        const float lin = rbf(sum);
-        if (which)
-            a.g[(size_t)t * Hv + h] = -expf(bf2f(a.a_log[h])) * softplusf_(lin + bf2f(a.dt_bias[h])) * valid;
-        else
-            a.beta[(size_t)t * Hv + h] = rbf(sigmoidf_(lin)) * valid;
-    }
-
-    // Channel ci of this block: q (0..127) and k (128..255) of key head kh, then v of its value heads.
-    auto mixed = [&](int ci) {
-        const int c = ci < D ? kh * D + ci : ci < 2 * D ? Hk * D + kh * D + ci - D : 2 * Hk * D + kh * rep * D + ci - 2 * D;
-        const bf16_t* wc = a.conv_w + (size_t)c * 4;
-        float m = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float p = rbf(conv_window(a, hist, keep, c, t + j) * bf2f(wc[j]));
-            m = j == 0 ? p : rbf(m + p);
-        }
-        return rbf(m * rbf(sigmoidf_(m)));
+    const int tw = t0 + 8 * wave;  // this wave's first token
+    // Inputs of head hd (q, k, then the value heads): the window of this wave's tokens, a word of two channels each, and the
+    // taps; the next head's load while this one's are used.
+    auto channel = [&](int hd) {
+        return (hd == 0 ? kh * D : hd == 1 ? Hk * D + kh * D : 2 * Hk * D + (kh * rep + hd - 2) * D) + 2 * lane;
     };
-
-    // q and k: one channel per thread, l2 norms over each 128 (waves 0-1: q, 2-3: k).
-    const float x = mixed(tid);
-    float ss = warp_sum(x * x);
-    if (lane == 0) red[wave] = ss;
+    uint32_t xw[11];
+    uint4 cw;
+    auto load = [&](int hd) {
+        const int c = channel(hd);
+#pragma unroll
+        for (int j = 0; j < 11; ++j)
+            xw[j] = j < 3 && tw == 0 ? pk_bf16(conv_window(a, hist, keep, c, j), conv_window(a, hist, keep, c + 1, j))
+                                     : *(const uint32_t*)(a.qkv + (size_t)(tw + j - 3) * C + c);
+        cw = *(const uint4*)(a.conv_w + (size_t)c * 4);
+    };
+    load(0);
+    for (int hd = 0; hd < 2 + rep; ++hd) {
+        float x[11][2];
+#pragma unroll
+        for (int j = 0; j < 11; ++j) x[j][0] = lo_bf(xw[j]), x[j][1] = hi_bf(xw[j]);
+        const float w[2][4] = {{lo_bf(cw.x), hi_bf(cw.x), lo_bf(cw.y), hi_bf(cw.y)}, {lo_bf(cw.z), hi_bf(cw.z), lo_bf(cw.w), hi_bf(cw.w)}};
+        if (hd + 1 < 2 + rep) load(hd + 1);
+        float y[8][2];
+        auto round2 = [](float& p, float& q) {  // both to bf16 and back, one conversion
+            const uint32_t r = pk_bf16(p, q);
+            p = lo_bf(r);
+            q = hi_bf(r);
+        };
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            float m[2];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {  // bf16 tap products summed by bf16 additions (model.py:514)
+                float p[2] = {x[t + j][0] * w[0][j], x[t + j][1] * w[1][j]};
+                round2(p[0], p[1]);
+                m[0] = j ? m[0] + p[0] : p[0];
+                m[1] = j ? m[1] + p[1] : p[1];
+                if (j) round2(m[0], m[1]);
+            }
+            float g[2] = {sigmoidf_(m[0]), sigmoidf_(m[1])};
+            round2(g[0], g[1]);
+            y[t][0] = m[0] * g[0];
+            y[t][1] = m[1] * g[1];
+            round2(y[t][0], y[t][1]);
+        }
+        if (hd < 2) {
+            float ss[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) ss[t] = y[t][0] * y[t][0] + y[t][1] * y[t][1];
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+                for (int t = 0; t < 8; ++t) ss[t] += __shfl_xor(ss[t], o);
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                const float rs = 1.0f / sqrtf(ss[t] + 1e-6f);
+                const float2 v = hd ? make_float2(y[t][0] * rs, y[t][1] * rs)
+                                    : make_float2((y[t][0] * rs) / 11.313708498984761f, (y[t][1] * rs) / 11.313708498984761f);
+                *(float2*)((hd ? a.kn : a.qn) + ((size_t)(tw + t) * Hk + kh) * D + 2 * lane) = v;
+                *(float2*)&(hd ? sk : sq)[8 * wave + t][2 * lane] = v;
+            }
+        } else {
+            const int h = kh * rep + hd - 2;
+#pragma unroll
+            for (int t = 0; t < 8; ++t) *(uint32_t*)(a.v + ((size_t)(tw + t) * Hv + h) * D + 2 * lane) = pk_bf16(y[t][0], y[t][1]);
+        }
+    }
     __syncthreads();
-    const float tot = wave < 2 ? red[0] + red[1] : red[2] + red[3];
-    const float rs = 1.0f / sqrtf(tot + 1e-6f);
-    if (wave < 2)
-        a.qn[((size_t)t * Hk + kh) * D + tid] = (x * rs) / 11.313708498984761f;
-    else
-        a.kn[((size_t)t * Hk + kh) * D + tid - D] = x * rs;
-    // v of the rep value heads.
-    for (int ci = 2 * D + tid; ci < (2 + rep) * D; ci += 256) {
-        const int h = kh * rep + (ci - 2 * D) / D, d = (ci - 2 * D) % D;
-        a.v[((size_t)t * Hv + h) * D + d] = mixed(ci);
+
+    // k . k and q . k, a 16 x 16 quarter per wave (rows t, columns s; the quarter above the diagonal stays zero): four
+    // MFMA steps per 16-byte read, the same order of inputs in both operands.
+    const int wr = wave >> 1, wc = wave & 1, lr = lane & 15, lq = lane >> 4;
+    v4f kk = {0.0f, 0.0f, 0.0f, 0.0f}, qk = kk;
+    if (wr >= wc)
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+            const v4f kt = *(const v4f*)&sk[16 * wr + lr][16 * g + 4 * lq], qt = *(const v4f*)&sq[16 * wr + lr][16 * g + 4 * lq];
+            const v4f ks = *(const v4f*)&sk[16 * wc + lr][16 * g + 4 * lq];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                kk = mfma16(kt[e], ks[e], kk);
+                qk = mfma16(qt[e], ks[e], qk);
+            }
+        }
+    for (int r0 = 0; r0 < rep; r0 += 4) {  // value heads, four at a time
+        const int nh = min(4, rep - r0);
+        // Gates (model.py:333-337, 499-500), then the chunk's cumulative log decays: a half wave per head.
+        if (tid < 32 * nh) {
+            const int r = tid >> 5, t = t0 + (tid & 31), h = kh * rep + r0 + r, O = 2 * Hv;
+            const float valid = t < nv ? 1.0f : 0.0f;
+            float sum[2] = {0.0f, 0.0f};
+#pragma unroll
+            for (int gi = 0; gi < GMAX; ++gi)
+                if (gi < a.gate_groups) {
+                    const float* p = a.gate_part + ((size_t)gi * a.L + t) * O + h;
+                    sum[0] += p[0];
+                    sum[1] += p[Hv];
+                }
+            const float beta = rbf(sigmoidf_(rbf(sum[0]))) * valid;
+            // Summed in 64 bits: the factors are e to differences of these sums, often small ones of large ones.
+            double c = -expf(bf2f(a.a_log[h])) * softplusf_(rbf(sum[1]) + bf2f(a.dt_bias[h])) * valid;
+#pragma unroll
+            for (int o = 1; o < 32; o <<= 1) {
+                const double up = __shfl_up(c, o, 32);
+                if ((tid & 31) >= o) c += up;
+            }
+            sb[r][tid & 31] = beta;
+            sc[r][tid & 31] = c;
+            const double last = __shfl(c, 31, 32) - c;
+            float* f = a.decay + (((size_t)ch * Hv + h) * 3) * GC + (tid & 31);
+            f[0] = beta;
+            f[GC] = exp_of(c);
+            f[2 * GC] = exp_of(last);
+        }
+        __syncthreads();
+        for (int r = 0; r < nh; ++r) {
+            float* P = a.pt + ((size_t)ch * Hv + kh * rep + r0 + r) * 2 * GC * GC + GC * GC;
+            const int s = 16 * wc + lr;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int t = 16 * wr + 4 * lq + i;
+                const float e = t >= s ? exp_of(sc[r][t] - sc[r][s]) : 0.0f;
+                sm[r][t][s] = sb[r][t] * e * kk[i];
+                P[t * GC + s] = e * qk[i];
+            }
+        }
+        __syncthreads();
+        if (wave < nh && lane < GC) {  // column `lane` of T
+            float* T = a.pt + ((size_t)ch * Hv + kh * rep + r0 + wave) * 2 * GC * GC;
+            float col[GC];
+#pragma unroll
+            for (int i = 0; i < GC; ++i) {
+                float v = i == lane ? 1.0f : 0.0f;
+#pragma unroll
+                for (int s4 = 0; s4 < i; s4 += 4) {
+                    const v4f m = *(const v4f*)&sm[wave][i][s4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (s4 + e < i) v -= m[e] * col[s4 + e];
+                }
+                col[i] = v;
+                T[i * GC + lane] = v;
+            }
+        }
+        if (r0 + 4 < rep) __syncthreads();  // sm, sb and sc are read before the next heads' are written
     }
 }
 
-// Grid (value head, group of 32 state columns); thread (column c = tid / 8, rows 16 (tid % 8) + [0, 16)). Tokens are
-// staged through LDS 16 at a time in two buffers: each round's loads are issued into registers before the round
-// before it runs, so their latency hides behind its 16 token steps.
+// The delta rule over the chunks, grid (value head, group of 32 state columns), four waves. The state S (128 x 32 here)
+// stays in registers, wave w rows 32 w .. 32 w + 31 as one 32x32 float32 accumulator, whose registers are at the same
+// time the B operands of the next chunk's reads (MFMA i takes state rows drow(i, half)). Per chunk of 32 tokens:
+//   k . S and q . S over the wave's rows, the four waves' parts added through LDS;  R = beta (v - e^c k . S)
+//   Delta = T R;  o = e^c q . S + P Delta;  S = e^(c_last) S + (e^(c_last - c) k)^T Delta
+// all in float32 on the float32 MFMA. The reference runs the same in pieces of 128 tokens (chunked_gated_delta,
+// model.py:88-124); 32 keep T and P small, and the state's products, which are most of the work, do not depend on it.
+// Bounds: the float32 matrix rate of the CUs that 4 Hv workgroups fill: per wave and chunk 32 + 16 MFMAs of 64 cycles and
+// 16 of 32, with three LDS round trips between them. k, q, T, P, v and the gates of the next chunk load meanwhile.
+// 2,048 tokens of the 27B layer (64 chunks): 218 us, 49 TFLOP/s; token by token (one state column in 8 lanes, DPP
+// sums) 781 us. Against 64 bits from the same k, q, v, beta and g, o before its rounding to bf16 is off by
+// 1.8e-7 (1.0e-7 token by token) and after it by 1.658e-3, the state by 1.66e-3, as before.
 __global__ __launch_bounds__(256) void gdn_prefill_scan_kernel(const PrefillGdnArgs a) {
-    constexpr int D = 128, TB = 16;  // tokens staged per round
-    __shared__ __attribute__((aligned(16))) float sk[2][TB][D], sq[2][TB][D];
-    __shared__ float sv[2][TB][32], sb[2][TB], sg[2][TB];
-    const int h = blockIdx.x, grp = blockIdx.y, tid = threadIdx.x;
-    const int Hk = a.Hk, Hv = a.Hv, kh = h / (Hv / Hk);
-    const int c = tid >> 3, r = tid & 7, j = grp * 32 + c, i0 = r * 16;
+    constexpr int D = 128, KB = GC * D * 4, RP = 36;  // bytes of a chunk's k or q, floats per row of the 32 x 32 tiles
+    __shared__ __attribute__((aligned(1024))) uint8_t ring[2][2][KB];  // [stage][k, q], 16-byte chunk c of row r at c ^ (r % 16)
+    __shared__ __attribute__((aligned(16))) float red[4][2][4][64][4];
+    __shared__ __attribute__((aligned(16))) float sR[GC][RP], sO[GC][RP], sD[GC][RP], sW[GC][RP];
+    __shared__ float sf[2][3 * GC];  // beta, e^c, e^(c_last - c), by chunk parity: a chunk's tail reads while the next's are written
+    const int h = blockIdx.x, grp = blockIdx.y, tid = threadIdx.x, lane = tid & 63, hf = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int Hk = a.Hk, Hv = a.Hv, kh = h / (Hv / Hk), nch = a.L / GC;
     const int slot = *a.slot;
     if (slot < 0 || slot >= a.rows) return;
     const float keep = *a.start > 0 ? 1.0f : 0.0f;
-    bf16_t* st = a.state + ((size_t)slot * Hv + h) * D * D;
-    float s[16];
+    bf16_t* st = a.state + ((size_t)slot * Hv + h) * D * D + grp * 32 + (lane & 31);
+    auto row = [&](int i) { return 32 * wave + 8 * (i >> 2) + 4 * hf + (i & 3); };
+    v16f S;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) s[e] = bf2f(st[(size_t)(i0 + e) * D + j]) * keep;
+    for (int i = 0; i < 16; ++i) S[i] = bf2f(st[(size_t)row(i) * D]) * keep;
 
-    // One round's loads: 2 float4 of k and of q, 2 values of v, and beta and g for threads 0 .. TB - 1; tokens past
-    // the chunk load its last token (never used).
-    static_assert(TB * D / 4 == 2 * 256 && TB * 32 == 2 * 256, "two pieces per thread");
-    float4 rk[2], rq[2];
-    float rv[2], rb = 0.0f, rg = 0.0f;
-    auto load = [&](int t0) {
+    // Loads of chunk c: k and q into stage c % 2 (a wave 8 rows of each, two per instruction), T's and P's rows of this
+    // wave's quarter, the four v of this thread's tokens 8 w + 4 hf + e, and for threads 0..95 the tokens' factors.
+    const int wr = wave >> 1, wc = wave & 1, lr = lane & 15, lq = lane >> 4;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)LDS_PTR(&ring[0][0][0]);
+    v4f T[2], P[2];
+    uint32_t vr[4];
+    float gf = 0.0f;
+    auto load = [&](int c) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int e = tid + 256 * u, t = min(t0 + e / (D / 4), a.L - 1), d = (e % (D / 4)) * 4;
-            rk[u] = *(const float4*)(a.kn + ((size_t)t * Hk + kh) * D + d);
-            rq[u] = *(const float4*)(a.qn + ((size_t)t * Hk + kh) * D + d);
-            const int tv = min(t0 + e / 32, a.L - 1);
-            rv[u] = a.v[((size_t)tv * Hv + h) * D + grp * 32 + e % 32];
+        for (int w = 0; w < 2; ++w) {
+            const uint8_t* src = (const uint8_t*)(w ? a.qn : a.kn) + ((size_t)c * GC * Hk + kh) * D * 4;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int r = 8 * wave + 2 * j + hf;
+                lds_quad(src, (uint32_t)(r * Hk * D * 4 + (((lane & 31) ^ (r & 15)) << 4)),
+                         lds0 + ((c & 1) * 2 + w) * KB + (8 * wave + 2 * j) * D * 4);
+            }
         }
-        const int tb = min(t0 + (tid & (TB - 1)), a.L - 1);
-        rb = a.beta[(size_t)tb * Hv + h];
-        rg = a.g[(size_t)tb * Hv + h];
+        const float* pt = a.pt + ((size_t)c * Hv + h) * 2 * GC * GC + (16 * wr + lr) * GC + 4 * lq;
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            T[g] = *(const v4f*)(pt + 16 * g);
+            P[g] = *(const v4f*)(pt + GC * GC + 16 * g);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            vr[e] = a.v[((size_t)(c * GC + 8 * wave + 4 * hf + e) * Hv + h) * D + grp * 32 + (lane & 31)];
+        if (tid < 3 * GC) gf = a.decay[((size_t)c * Hv + h) * 3 * GC + tid];
     };
     load(0);
-    for (int t0 = 0, buf = 0; t0 < a.L; t0 += TB, buf ^= 1) {
-        // Buffer buf was last read two rounds ago, before every thread passed the last round's barrier.
+    for (int c = 0; c < nch; ++c) {
+        // Everything but the last chunk's four output stores.
+        if (c == 0)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        const float *sb = sf[c & 1], *se = sb + GC, *sw = sb + 2 * GC;
+        if (tid < 3 * GC) sf[c & 1][tid] = gf;
+        const v4f Tc[2] = {T[0], T[1]}, Pc[2] = {P[0], P[1]};
+        float vc[4];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int e = tid + 256 * u, tt = e / (D / 4), d = (e % (D / 4)) * 4;
-            *(float4*)&sk[buf][tt][d] = rk[u];
-            *(float4*)&sq[buf][tt][d] = rq[u];
-            sv[buf][e / 32][e % 32] = rv[u];
+        for (int e = 0; e < 4; ++e) vc[e] = __uint_as_float(vr[e] << 16);
+        lds_barrier();  // the chunk's k, q and gates are in LDS; every wave is done with the chunk before
+        // This wave's LDS operands of k . S, q . S and the state's update (rows of k down its 32 columns) in one go: read
+        // one by one before their MFMAs they cost their latency each. The fences keep the reads here.
+        const uint32_t kq = lds0 + (c & 1) * 2 * KB;
+        auto piece = [&](uint32_t base, int g) __attribute__((always_inline)) {  // inputs 32 w + 8 g + 4 hf + [0, 4) of token lane % 32
+            const int r = lane & 31;
+            return *(const __attribute__((address_space(3))) v4f*)(uintptr_t)(base + r * D * 4 + (((8 * wave + 2 * g + hf) ^ (r & 15)) << 4));
+        };
+        v4f kp[4], qp[4];
+        float kt[16];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) kp[g] = piece(kq, g), qp[g] = piece(kq + KB, g);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int s = 2 * j + hf;
+            kt[j] = *(const __attribute__((address_space(3))) float*)(uintptr_t)(
+                kq + s * D * 4 + (((8 * wave + ((lane & 31) >> 2)) ^ (s & 15)) << 4) + (lane & 3) * 4);
         }
-        if (tid < TB) {
-            sb[buf][tid] = rb;
-            sg[buf][tid] = rg;
+        __builtin_amdgcn_sched_barrier(0);
+        if (c + 1 < nch) load(c + 1);
+
+        // k . S and q . S over this wave's 32 state rows.
+        v16f ks, qs;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) ks[i] = qs[i] = 0.0f;
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                ks = __builtin_amdgcn_mfma_f32_32x32x2f32(kp[g][e], S[4 * g + e], ks, 0, 0, 0);
+                qs = __builtin_amdgcn_mfma_f32_32x32x2f32(qp[g][e], S[4 * g + e], qs, 0, 0, 0);
+            }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            *(v4f*)red[wave][0][q][lane] = (v4f){ks[4 * q], ks[4 * q + 1], ks[4 * q + 2], ks[4 * q + 3]};
+            *(v4f*)red[wave][1][q][lane] = (v4f){qs[4 * q], qs[4 * q + 1], qs[4 * q + 2], qs[4 * q + 3]};
         }
-        __syncthreads();
-        if (t0 + TB < a.L) load(t0 + TB);
-        const int nt = min(TB, a.L - t0);
-        for (int tt = 0; tt < nt; ++tt) {
-            const float e = expf(sg[buf][tt]);
-            float kv[16], qv[16];
+        lds_barrier();
+        {  // this thread: tokens 8 w + 4 hf + e, column lane % 32
+            v4f kw[4], qw[4];
 #pragma unroll
-            for (int q = 0; q < 16; q += 4) {
-                *(float4*)&kv[q] = *(const float4*)&sk[buf][tt][i0 + q];
-                *(float4*)&qv[q] = *(const float4*)&sq[buf][tt][i0 + q];
-            }
-            float ks = 0.0f;
+            for (int w = 0; w < 4; ++w) kw[w] = *(const v4f*)red[w][0][wave][lane], qw[w] = *(const v4f*)red[w][1][wave][lane];
+            __builtin_amdgcn_sched_barrier(0);
+            const v4f k4 = (kw[0] + kw[1]) + (kw[2] + kw[3]), q4 = (qw[0] + qw[1]) + (qw[2] + qw[3]);
 #pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                s[q] *= e;
-                ks += s[q] * kv[q];
+            for (int e = 0; e < 4; ++e) {
+                const int t = 8 * wave + 4 * hf + e;
+                sR[t][lane & 31] = sb[t] * (vc[e] - se[t] * k4[e]);
+                sO[t][lane & 31] = se[t] * q4[e];
             }
-            ks = group8_sum(ks);
-            const float delta = (sv[buf][tt][c] - ks) * sb[buf][tt];
-            float os = 0.0f;
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                s[q] += kv[q] * delta;
-                os += s[q] * qv[q];
-            }
-            os = group8_sum(os);
-            if (r == 0) a.o[((size_t)(t0 + tt) * Hv + h) * D + j] = os;
         }
+        lds_barrier();
+        // Delta, a 16 x 16 quarter per wave (T is lower triangular: the upper quarters sum 16 tokens).
+        float rr[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) rr[j] = sR[16 * (j >> 2) + 4 * lq + (j & 3)][16 * wc + lr];
+        __builtin_amdgcn_sched_barrier(0);
+        v4f dl = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dl = mfma16(Tc[0][e], rr[e], dl);
+        if (wr)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dl = mfma16(Tc[1][e], rr[4 + e], dl);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int t = 16 * wr + 4 * lq + i;
+            sD[t][16 * wc + lr] = dl[i];
+            sW[t][16 * wc + lr] = dl[i] * sw[t];
+        }
+        const float es = se[GC - 1];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) S[i] *= es;
+        lds_barrier();
+        // The state, and beside its chain the outputs.
+        float dw[16], dd[8];
+        v4f oq;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) dw[j] = sW[2 * j + hf][lane & 31];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) dd[j] = sD[16 * (j >> 2) + 4 * lq + (j & 3)][16 * wc + lr];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) oq[i] = sO[16 * wr + 4 * lq + i][16 * wc + lr];
+        __builtin_amdgcn_sched_barrier(0);
+        v4f op[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            S = __builtin_amdgcn_mfma_f32_32x32x2f32(kt[j], dw[j], S, 0, 0, 0);
+            if (j < 8) op[j >> 2] = mfma16(Pc[j >> 2][j & 3], dd[j], op[j >> 2]);
+        }
+        const v4f o = oq + (op[0] + op[1]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            a.o[((size_t)(c * GC + 16 * wr + 4 * lq + i) * Hv + h) * D + grp * 32 + 16 * wc + lr] = f2bf(o[i]);
     }
 #pragma unroll
-    for (int e = 0; e < 16; ++e) st[(size_t)(i0 + e) * D + j] = f2bf(s[e]);
+    for (int i = 0; i < 16; ++i) st[(size_t)row(i) * D] = f2bf(S[i]);
 }
 
-// Grid (token, value heads / 4): wave w takes value head 4 blockIdx.y + w (model.py:339-345).
+// The gated norm and out_proj's e5m2 tiles (model.py:339-345), grid (4 tokens, value heads / 4): wave w takes value head
+// 4 blockIdx.y + w, 16 lanes per token, 8 dims per lane: whole cache lines of o and z, 8-byte tile stores (one byte at a
+// time it took 40 us for 2,048 tokens of the 27B layer, 18 us now).
 __global__ __launch_bounds__(256) void gdn_prefill_finish_kernel(const PrefillGdnArgs a) {
     constexpr int D = 128;
-    const int t = blockIdx.x, lane = threadIdx.x & 63, h = blockIdx.y * 4 + (threadIdx.x >> 6);
-    const int Hv = a.Hv;
-    if (h >= Hv) return;
-    const float o0 = rbf(a.o[((size_t)t * Hv + h) * D + lane]), o1 = rbf(a.o[((size_t)t * Hv + h) * D + lane + 64]);
-    const float r = 1.0f / sqrtf(warp_sum(o0 * o0 + o1 * o1) / 128.0f + a.eps);
+    const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (lane >> 4), d = (lane & 15) * 8;
+    const int h = blockIdx.y * 4 + (threadIdx.x >> 6), Hv = a.Hv;
+    const size_t at = ((size_t)t * Hv + h) * D + d;
+    const uint4 ow = *(const uint4*)(a.o + at), zw = *(const uint4*)(a.z + at), nw = *(const uint4*)(a.norm_w + d);
+    const uint32_t o2[4] = {ow.x, ow.y, ow.z, ow.w}, z2[4] = {zw.x, zw.y, zw.z, zw.w}, n2[4] = {nw.x, nw.y, nw.z, nw.w};
+    float o[8], ss = 0.0f;
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-        const int jj = lane + half * 64;
-        float hv = rbf((half ? o1 : o0) * r);
-        hv = rbf(bf2f(a.norm_w[jj]) * hv);
-        const float zf = bf2f(a.z[(size_t)t * Hv * D + h * D + jj]);
-        a.act[act_offset(t, h * D + jj, Hv * D)] = (uint8_t)e5m2_byte(rbf(hv * (zf * sigmoidf_(zf))));
+    for (int e = 0; e < 8; ++e) {
+        o[e] = e & 1 ? hi_bf(o2[e >> 1]) : lo_bf(o2[e >> 1]);
+        ss += o[e] * o[e];
     }
+    const float r = 1.0f / sqrtf(group16_sum(ss) / 128.0f + a.eps);
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float z = e & 1 ? hi_bf(z2[e >> 1]) : lo_bf(z2[e >> 1]), n = e & 1 ? hi_bf(n2[e >> 1]) : lo_bf(n2[e >> 1]);
+        v[e] = rbf(rbf(n * rbf(o[e] * r)) * (z * sigmoidf_(z)));
+    }
+    *(uint2*)(a.act + act_offset(t, h * D + d, Hv * D)) = make_uint2(pk_e5m2(v[0], v[1], v[2], v[3]), pk_e5m2(v[4], v[5], v[6], v[7]));
 }
 
 // The row's new conv state (model.py:492-495): inputs n_valid .. n_valid + 2 of [history * keep, chunk].
@@ -401,12 +630,6 @@ __device__ __forceinline__ size_t prefill_slot(const PrefillAttnArgs& a, int kvh
 }
 
 __device__ __forceinline__ float order_float(int i) { return __int_as_float(i >= 0 ? i : i ^ 0x7fffffff); }
-
-// 16 bytes per lane from base + off (base wave-uniform) to LDS dst + 16 l (dst wave-uniform), as lds_dword.
-__device__ __forceinline__ void lds_quad(const void* base, uint32_t off, uint32_t dst) {
-    const uint32_t m0 = __builtin_amdgcn_readfirstlane(dst);
-    asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(m0) : "memory");
-}
 
 __device__ __forceinline__ v8bf16 lds_frag(uint32_t at) {
     return *(const __attribute__((address_space(3))) v8bf16*)(uintptr_t)at;
@@ -811,9 +1034,10 @@ hipError_t q38_attn_prefill(const PrefillAttnArgs& a0, hipStream_t stream) {
 hipError_t q38_gdn_prefill(const PrefillGdnArgs& a, hipStream_t stream) {
     if (a.L < 1 || a.gate_groups < 1 || a.gate_groups > 8 || a.Hv % a.Hk || a.Hv % 4 || a.C != 2 * a.Hk * 128 + a.Hv * 128)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(gdn_prefill_prep_kernel, dim3(a.L, a.Hk), dim3(256), 0, stream, a);
+    if (a.L % GC || a.Hv % 4) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(gdn_prefill_prep_kernel, dim3(a.L / GC, a.Hk), dim3(256), 0, stream, a);
     hipLaunchKernelGGL(gdn_prefill_scan_kernel, dim3(a.Hv, 4), dim3(256), 0, stream, a);
-    hipLaunchKernelGGL(gdn_prefill_finish_kernel, dim3(a.L, a.Hv / 4), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(gdn_prefill_finish_kernel, dim3(a.L / 4, a.Hv / 4), dim3(256), 0, stream, a);
     hipLaunchKernelGGL(gdn_prefill_carry_kernel, dim3((a.C + 255) / 256), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
