@@ -32,6 +32,9 @@
 //                projection's activation tiles (the chip's fused mlp_up, kernels.py:74-118)
 //   EPI_PARTIAL  float32 partial sums [split][Tpad][N]
 //   EPI_GROUPMAX largest float32 logit of each 32-row tile per token (the head's group maxima, kernels.py:126-172)
+#include <algorithm>
+#include <type_traits>
+
 #include "kernels.h"
 
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
@@ -633,6 +636,265 @@ __global__ __launch_bounds__(WF * WT * 64, 1) void gemm_kernel(const GemmArgs a)
     }
 }
 
+// Up to 64 tokens: a weight-streaming kernel, bound by HBM. A workgroup of KW waves works on 64 features; its waves split
+// the K range and each takes all tokens, so nothing is shared between waves before a tile's end: weights, scales and
+// activations go straight to registers, D K-steps ahead (a K-step is 4 KiB of e4m3 weights per wave), with no ring and no
+// barrier; at the end the waves' sums are added in K order through LDS, one feature tile at a time, with the next tile's
+// first loads in flight. (With 128 to 512 features per workgroup in the ring kernel, a tile's K range was split over up
+// to twelve workgroups whose parts the last one added one after another, and every K-step met a barrier.)
+//
+// Schedule. What counts is that every CU moves the same bytes, and that few tiles are split. Of the tiles, whole multiples of
+// the CUs are one workgroup's each; the rest are split in K over `splits` workgroups on one XCD each, as many as the CUs
+// take, finished by the last to arrive from the others' sums in that XCD's L2 (or, should one have run elsewhere, by
+// computing theirs again). EPI_PARTIAL: K split over workgroups, a part each.
+template <int TT, int EPI, bool W4, int KW>
+__global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(2))) void gemm_stream_kernel(const GemmArgs a) {
+    constexpr int FR = 2, WTB = W4 ? 1024 : 2048;
+    constexpr int D = TT == 1 ? 4 : 3;  // K-steps in flight
+    static_assert(D * (5 * FR + 4 * TT) <= 63, "vmcnt range");
+    constexpr int G = TT * 4, GW = (G + KW - 1) / KW;  // (token tile, quarter of the rows) quads of a feature tile, per wave
+    __shared__ __attribute__((aligned(16))) float red[KW * G * 256];
+    __shared__ unsigned long long s_arrived;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tiles = a.N / (32 * FR), KS = a.K >> 6;
+
+    struct Seg {
+        int fb, k0, k1;  // K-steps [k0, k1) of tile fb
+    };
+    typedef typename std::conditional<W4, uint32_t, u2>::type WFrag;
+    struct Step {
+        WFrag w[FR][4];
+        u2 x[TT][4];
+        uint16_t sc[FR];
+    };
+    Step st[D];
+    // This wave's part of a segment's K range.
+    auto part0 = [&](const Seg& s, int w) { return s.k0 + (int)((long)w * (s.k1 - s.k0) / KW); };
+    auto load = [&](int fb, int k, Step& s) __attribute__((always_inline)) {
+        k = min(k, KS - 1);  // past the range: loaded, never used
+        const uint8_t* wp = a.w + ((size_t)(fb * FR) * KS + k) * WTB;
+        const uint8_t* sp = a.ws + ((size_t)(fb * FR) * KS + k) * 64;
+        const uint8_t* xp = (const uint8_t*)a.act + (size_t)k * 2048;
+#pragma unroll
+        for (int f = 0; f < FR; ++f) {
+            s.sc[f] = *(const uint16_t*)(sp + (size_t)f * KS * 64 + (lane & 31) * 2);
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+                s.w[f][m] = __builtin_nontemporal_load((const WFrag*)(wp + (size_t)f * KS * WTB + m * (WTB / 4) + lane * (WTB / 256)));
+        }
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) s.x[t][m] = *(const u2*)(xp + (size_t)t * KS * 2048 + m * 512 + lane * 8);
+    };
+    v16f acc[FR][TT];
+    auto compute = [&](const Step& s) __attribute__((always_inline)) {
+        float scl[FR][2];
+#pragma unroll
+        for (int f = 0; f < FR; ++f) {
+            scl[f][0] = __uint_as_float((uint32_t)(s.sc[f] & 0xff) << 23);
+            scl[f][1] = __uint_as_float((uint32_t)(s.sc[f] >> 8) << 23);
+        }
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            v8bf wb[FR], xb[TT];
+#pragma unroll
+            for (int f = 0; f < FR; ++f) {
+                if constexpr (W4)
+                    wb[f] = widen_e2m1(s.w[f][m], scl[f][m >> 1]);
+                else
+                    wb[f] = widen_e4m3(s.w[f][m][0], s.w[f][m][1], scl[f][m >> 1]);
+            }
+#pragma unroll
+            for (int t = 0; t < TT; ++t) xb[t] = widen_e5m2(s.x[t][m][0], s.x[t][m][1]);
+#pragma unroll
+            for (int f = 0; f < FR; ++f)
+#pragma unroll
+                for (int t = 0; t < TT; ++t) acc[f][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wb[f], xb[t], acc[f][t], 0, 0, 0);
+        }
+    };
+    auto fill = [&](const Seg& s) __attribute__((always_inline)) {
+        const int k = part0(s, wave);
+#pragma unroll
+        for (int d = 0; d < D; ++d) load(s.fb, k + d, st[d]);
+    };
+    // The segment's products over this wave's K range, its first D K-steps already on their way.
+    auto run = [&](const Seg& s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int f = 0; f < FR; ++f)
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[f][t][i] = 0.0f;
+        int k = part0(s, wave);
+        const int k1 = part0(s, wave + 1);
+        for (; k + D <= k1; k += D) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                compute(st[d]);
+                load(s.fb, k + D + d, st[d]);
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < D - 1; ++d)
+            if (k + d < k1) compute(st[d]);
+    };
+    // The waves' sums added in K order, a feature tile at a time; wave w then holds quads w, w + KW, ...: features
+    // 8 q + 4 (l / 32) + [0, 4) of token 32 t + l % 32 for quad 4 t + q.
+    v4f sum[FR][GW];
+    auto lds_sync = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };  // loads stay in flight
+    auto reduce = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int f = 0; f < FR; ++f) {
+            lds_sync();  // the last reads of red are done
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *(v4f*)(red + ((wave * G + t * 4 + q) * 64 + lane) * 4) =
+                        (v4f){acc[f][t][4 * q], acc[f][t][4 * q + 1], acc[f][t][4 * q + 2], acc[f][t][4 * q + 3]};
+            lds_sync();
+#pragma unroll
+            for (int j = 0; j < GW; ++j) {
+                const int g = wave + j * KW;
+                if (g < G) {
+                    v4f x[KW];
+#pragma unroll
+                    for (int w = 0; w < KW; ++w) x[w] = *(const v4f*)(red + ((w * G + g) * 64 + lane) * 4);
+#pragma unroll
+                    for (int w = 1; w < KW; ++w) x[0] += x[w];
+                    sum[f][j] = x[0];
+                }
+            }
+        }
+    };
+    auto epilogue = [&](int fb, int z) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < GW; ++j) {
+            const int g = wave + j * KW;
+            if (g >= G) break;
+            const int tok = (g >> 2) * 32 + (lane & 31), row = (g & 3) * 8 + (lane >> 5) * 4;
+            if constexpr (EPI == EPI_SWIGLU) {
+                float h[4];  // the two feature tiles: gate and up of the same 32 inner features
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float gv = rbf(sum[0][j][e]), uv = rbf(sum[1][j][e]);
+                    h[e] = rbf(rbf(gv * rbf(sigmoidf_(gv))) * uv);
+                }
+                *(uint32_t*)((uint8_t*)a.out0 + act_offset(tok, fb * 32 + row, a.N >> 1)) = pk_e5m2(h[0], h[1], h[2], h[3]);
+            } else {
+#pragma unroll
+                for (int f = 0; f < FR; ++f) {
+                    const int col = (fb * FR + f) * 32 + row;
+                    const v4f v = sum[f][j];
+                    if constexpr (EPI == EPI_PARTIAL) {
+                        *(v4f*)(a.part + ((size_t)z * a.Tpad + tok) * a.N + col) = v;
+                    } else if (tok < a.T) {
+                        bf16_t* dst = col < a.n0 ? (bf16_t*)a.out0 + (size_t)tok * a.ld0 + col
+                                                 : (bf16_t*)a.out1 + (size_t)tok * a.ld1 + (col - a.n0);
+                        *(uint2*)dst = make_uint2(pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3]));
+                    }
+                }
+            }
+        }
+    };
+
+    if constexpr (EPI == EPI_PARTIAL) {
+        const int z = blockIdx.x / tiles;
+        const Seg s = {(int)(blockIdx.x % tiles), z * KS / a.splits, (z + 1) * KS / a.splits};
+        fill(s);
+        run(s);
+        reduce();
+        epilogue(s.fb, z);
+    } else {
+        const int whole = tiles / a.cus * a.cus, i = (int)blockIdx.x - whole, n = i < 0 ? 1 : a.splits;
+        const int rest = (i >> 3) / n * 8 + (i & 7), z = (i >> 3) % n;  // among the split tiles, a tile's parts 8 ids apart
+        const int fb = i < 0 ? (int)blockIdx.x : whole + rest;
+        if (fb >= tiles) return;
+        auto part_of = [&](int p) { return Seg{fb, p * KS / n, (p + 1) * KS / n}; };
+        const Seg s = part_of(i < 0 ? 0 : z);
+        fill(s);
+        run(s);
+        reduce();
+        if (n > 1) {
+            uint32_t xcc_id;  // the XCD this workgroup actually runs on
+            asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc_id));
+            const unsigned long long own_byte = 0xffull << (8 * (xcc_id & 7));
+            constexpr int SLOT = FR * G * 256;  // floats of one part
+            auto slot_of = [&](int p) { return (size_t)(rest * n + p) * SLOT; };
+#pragma unroll
+            for (int f = 0; f < FR; ++f)
+#pragma unroll
+                for (int j = 0; j < GW; ++j)
+                    if (wave + j * KW < G) *(v4f*)(a.fix + slot_of(z) + ((f * G + wave + j * KW) * 64 + lane) * 4) = sum[f][j];
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (tid == 0)
+                s_arrived = __hip_atomic_fetch_add(a.counters + rest, own_byte & 0x0101010101010101ull, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            const unsigned long long others = s_arrived;
+            int arrived = 0;
+#pragma unroll
+            for (int x = 0; x < 8; ++x) arrived += (int)((others >> (8 * x)) & 0xff);
+            if (arrived != n - 1) return;
+            const bool again = a.recompute || (others & ~own_byte) != 0;
+            const __amdgpu_buffer_rsrc_t fix = __builtin_amdgcn_make_buffer_rsrc(a.fix, 0, 0x7fffffff, 0x00020000);
+            v4f total[FR][GW];
+#pragma unroll 1
+            for (int p = 0; p < n; ++p) {
+                if (again) {
+                    const Seg r = part_of(p);
+                    fill(r);
+                    run(r);
+                    reduce();
+                }
+#pragma unroll
+                for (int f = 0; f < FR; ++f)
+#pragma unroll
+                    for (int j = 0; j < GW; ++j) {
+                        if (wave + j * KW >= G) continue;
+                        if (!again)
+                            sum[f][j] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
+                                fix, (uint32_t)(slot_of(p) * 4) + ((f * G + wave + j * KW) * 64 + lane) * 16, 0, 1));
+                        total[f][j] = p ? total[f][j] + sum[f][j] : sum[f][j];
+                    }
+            }
+#pragma unroll
+            for (int f = 0; f < FR; ++f)
+#pragma unroll
+                for (int j = 0; j < GW; ++j) sum[f][j] = total[f][j];
+            if (tid == 0) __hip_atomic_store(a.counters + rest, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        epilogue(fb, 0);
+    }
+}
+
+// Waves per workgroup: eight, one workgroup per CU; four from two tiles per CU up, whose workgroups then share the CUs.
+// Splits: as many as the CUs take (of all tiles with EPI_PARTIAL, else of those beyond a multiple of the CUs), of at least
+// two K-steps per wave.
+template <int TT, int EPI, bool W4, int KW>
+hipError_t launch_stream(const GemmArgs& a0, int* splits_out, hipStream_t stream) {
+    GemmArgs a = a0;
+    const int tiles = a.N / 64, KS = a.K / 64, whole = EPI == EPI_PARTIAL ? 0 : tiles / a.cus * a.cus, rest = tiles - whole;
+    int s = std::min(std::min(rest ? a.cus / rest : 1, GEMM_SPLIT_MAX), KS / (2 * KW));
+    if (EPI == EPI_PARTIAL && a.splits_max > 0) s = std::min(s, a.splits_max);
+    a.splits = s = std::max(s, 1);
+    const int grid = EPI == EPI_PARTIAL ? tiles * s : whole + (rest + 7) / 8 * 8 * s;
+    if (EPI != EPI_PARTIAL && s > 1 && (rest > a.counters_n || (size_t)rest * s * 2 * TT * 1024 > a.fix_floats)) return hipErrorInvalidValue;
+    if (splits_out) *splits_out = EPI == EPI_PARTIAL ? s : 1;
+    hipLaunchKernelGGL((gemm_stream_kernel<TT, EPI, W4, KW>), dim3(grid), dim3(KW * 64), 0, stream, a);
+    return hipGetLastError();
+}
+
+template <int TT, int EPI, bool W4>
+hipError_t dispatch_stream(const GemmArgs& a, int* splits_out, hipStream_t stream) {
+    if (a.N % 64 || a.K % 64 || a.Tpad != 32 * TT || a.cus < 8 || a.cus % 8) return hipErrorInvalidValue;
+    if constexpr (EPI != EPI_PARTIAL)
+        if (a.N / 64 >= 2 * a.cus) return launch_stream<TT, EPI, W4, 4>(a, splits_out, stream);
+    return launch_stream<TT, EPI, W4, 8>(a, splits_out, stream);
+}
+
 constexpr int MIN_UNITS = 8;  // smallest K range worth a stream-K group
 
 template <int WF, int WT, int FR, int TR, bool A8, int S, int EPI, bool W4, bool F8, int KU = 1>
@@ -704,31 +966,43 @@ hipError_t dispatch(const GemmArgs& a, int* splits_out, hipStream_t stream) {
             return launch<4, 2, 2, 4, false, 3, EPI, W4, F8>(a, splits_out, stream);
         }
     }
+    // e5m2 activations up to 64 tokens stream their weights, but for the SwiGLU pair at 33 to 64 tokens: there the
+    // activations that every wave reads for itself weigh as much as the weights (gate/up of the 27B MLP 57 against 48.6 us
+    // e4m3, 49 against 42.7 us MXFP4; the bf16 outputs 23 against 28 and 17 against 26 us, the split-K partials 40 against
+    // 48.6 and 30 against 47 us; up to 32 tokens gate/up 42.7 against 45, bf16 outputs 19 against 35, partials 33 against 50).
+    constexpr bool RING32 = !A8 || F8, RING64 = RING32 || EPI == EPI_SWIGLU;
     const bool wide = a.N % 512 == 0 && (balanced(512) || !balanced(256));
     switch (a.Tpad) {
         case 128:
             return wide ? launch<8, 1, 2, 4, A8, 3, EPI, W4, F8>(a, splits_out, stream)
                         : launch<4, 2, 2, 2, A8, 3, EPI, W4, F8>(a, splits_out, stream);
         case 64:
-            // Measured per epilogue at 64 tokens (the decode step's projections): bf16 outputs fastest as 128 x 64
-            // tiles with a deep ring (qkvz 32 against 50 us as 512 x 64), split-K partials as 128 x 64 with 5 stages,
-            // the SwiGLU pair as 256 x 64 (50.9 against 56.4 us as 128 x 64).
-            if constexpr (A8) {
-                if (EPI == EPI_BF16 && balanced(128)) return launch<2, 2, 2, 1, true, 8, EPI, W4, F8>(a, splits_out, stream);
-                if (EPI == EPI_PARTIAL && balanced(128)) return launch<2, 2, 2, 1, true, 5, EPI, W4, F8>(a, splits_out, stream);
-                if (!balanced(512) && !balanced(256) && balanced(128)) return launch<2, 2, 2, 1, true, 5, EPI, W4, F8>(a, splits_out, stream);
+            if constexpr (RING64) {
+                // The FP8 MFMA's bf16 outputs as 128 x 64 tiles with a deep ring, its partials with 5 stages; the SwiGLU
+                // pair as 256 x 64 (50.9 against 56.4 us as 128 x 64).
+                if constexpr (A8) {
+                    if (EPI == EPI_BF16 && balanced(128)) return launch<2, 2, 2, 1, true, 8, EPI, W4, F8>(a, splits_out, stream);
+                    if (EPI == EPI_PARTIAL && balanced(128)) return launch<2, 2, 2, 1, true, 5, EPI, W4, F8>(a, splits_out, stream);
+                    if (!balanced(512) && !balanced(256) && balanced(128))
+                        return launch<2, 2, 2, 1, true, 5, EPI, W4, F8>(a, splits_out, stream);
+                }
+                // bf16 activations at 64 tokens (the draft heads' group maxima): 512 x 64 tiles, 64 x 64 per wave, when N
+                // allows (248.3 against 261.5 us as 256 x 64 with 64 x 32 per wave, per 1.31 GB launch).
+                if constexpr (!A8) {
+                    if (a.N % 512 == 0) return launch<8, 1, 2, 2, false, 3, EPI, W4, F8>(a, splits_out, stream);
+                    return launch<4, 2, 2, 1, false, 6, EPI, W4, F8>(a, splits_out, stream);
+                }
+                return wide ? launch<8, 1, 2, 2, A8, (A8 ? 4 : 3), EPI, W4, F8>(a, splits_out, stream)
+                            : launch<4, 2, 2, 1, A8, 4, EPI, W4, F8>(a, splits_out, stream);
+            } else {
+                return dispatch_stream<2, EPI, W4>(a, splits_out, stream);
             }
-            // bf16 activations at 64 tokens (the draft heads' group maxima): 512 x 64 tiles, 64 x 64 per wave, when N
-            // allows (248.3 against 261.5 us as 256 x 64 with 64 x 32 per wave, per 1.31 GB launch).
-            if constexpr (!A8) {
-                if (a.N % 512 == 0) return launch<8, 1, 2, 2, false, 3, EPI, W4, F8>(a, splits_out, stream);
-                return launch<4, 2, 2, 1, false, 6, EPI, W4, F8>(a, splits_out, stream);
-            }
-            return wide ? launch<8, 1, 2, 2, A8, (A8 ? 4 : 3), EPI, W4, F8>(a, splits_out, stream)
-                        : launch<4, 2, 2, 1, A8, 4, EPI, W4, F8>(a, splits_out, stream);
         case 32:
-            return wide ? launch<8, 1, 2, 1, A8, 4, EPI, W4, F8>(a, splits_out, stream)
-                        : launch<4, 1, 2, 1, A8, 4, EPI, W4, F8>(a, splits_out, stream);
+            if constexpr (RING32)
+                return wide ? launch<8, 1, 2, 1, A8, 4, EPI, W4, F8>(a, splits_out, stream)
+                            : launch<4, 1, 2, 1, A8, 4, EPI, W4, F8>(a, splits_out, stream);
+            else
+                return dispatch_stream<1, EPI, W4>(a, splits_out, stream);
         default:
             return hipErrorInvalidValue;
     }

@@ -69,10 +69,10 @@ int q38_fp8_linear_noalloc(const uint16_t* x, int rows, int k, const uint8_t* ti
     uint8_t* base = nullptr;
     if (scratch_on_current_device(&base)) return 1;
     hipStream_t stream = (hipStream_t)stream_;
-    // The arrival counters of every tile this call can use start at zero (tiles of 128 or more features, token blocks
-    // of 32 or more), cleared by a kernel on the caller's stream, so a captured call records no memset.
+    // The arrival counters this call can use (one per workgroup, at most two per CU) start at zero, cleared by a kernel on
+    // the caller's stream, so a captured call records no memset.
     unsigned long long* counters = (unsigned long long*)(base + NOALLOC_TILES);
-    const int used = n / 128 * 2 < GEMM_COUNTERS ? n / 128 * 2 : GEMM_COUNTERS;
+    const int used = 2 * NOALLOC_CUS;
     hipLaunchKernelGGL(clear_counters_kernel, dim3((used + 255) / 256), dim3(256), 0, stream, counters, used);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return q38_report((std::string("clear_counters_kernel: ") + hipGetErrorString(e)).c_str());

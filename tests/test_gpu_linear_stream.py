@@ -1,0 +1,77 @@
+"""The weight-streaming projection (up to 64 tokens) where its schedule can go wrong: K ranges shorter than a workgroup's
+waves, tiles left over beyond a multiple of the CUs split in K, four-wave workgroups, ragged tokens; e4m3 and MXFP4.
+
+Held against float64: half a bf16 ulp of the result for its rounding, plus 2^-20 of sum |x w| for the float32 sums (as the
+projection tests allow; measured about 1e-8). Finishing the split tiles by recomputing their parts gives the same bits."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from qwen38_amd import ext
+from qwen38_amd.quant import dequantize_e4m3, dequantize_mxfp4, quantize_e4m3, quantize_mxfp4, round_e5m2
+
+
+def inputs(rows, k, n, mx):
+    g = torch.Generator(device="cuda").manual_seed(rows * 31 + k + n)
+    w = torch.randn(n, k, generator=g, device="cuda") * 0.02
+    w[:, :32] *= 50.0  # groups with different scales
+    x = torch.randn(rows, k, generator=g, device="cuda").to(torch.bfloat16)
+    packed = quantize_mxfp4(w) if mx else quantize_e4m3(w)
+    return x, packed, (dequantize_mxfp4 if mx else dequantize_e4m3)(*packed).double()
+
+
+def check(got, x, wd):
+    xq = round_e5m2(x).double()
+    exact, bound = xq @ wd.T, (xq.abs() @ wd.abs().T) * 2.0**-20
+    ulp = torch.exp2(torch.floor(torch.log2(exact.abs().clamp_min(2.0**-126))) - 7)
+    off = (got.double() - exact).abs() - bound
+    assert bool((off <= ulp * 0.5 + bound).all()), float((off / ulp).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mx", [False, True])
+@pytest.mark.parametrize(
+    "rows, k, n",
+    [
+        (1, 256, 256),  # 4 tiles of 4 K-steps: most waves have none
+        (32, 768, 512),  # 12 K-steps over 8 waves
+        (33, 4352, 256),  # 4 tiles split 4 ways
+        (5, 1280, 16640),  # 256 whole tiles and 4 left over
+        (64, 512, 16640),
+        (17, 320 * 4, 33280),  # 520 tiles: four-wave workgroups, 8 left over
+        (61, 17408, 5120),  # 80 tiles split 3 ways
+    ],
+)
+def test_streamed_projection(gpu, rows, k, n, mx):
+    x, packed, wd = inputs(rows, k, n, mx)
+    if mx:
+        check(ext.mxfp4_linear(x, *ext.pack_weight_fp4(*packed), n), x, wd)
+        return
+    tiles, scales = ext.pack_weight(*packed)
+    got = ext.fp8_linear(x, tiles, scales, n)
+    check(got, x, wd)
+    again = ext.fp8_linear_mfma(x, tiles, scales, n, "bf16", recompute=True)
+    assert torch.equal(got.view(torch.int16), again.view(torch.int16))
+    scratch = ext.linear_scratch(rows, k)
+    for _ in range(2):  # the arrival counters are zero again after a call
+        assert torch.equal(ext.fp8_linear(x, tiles, scales, n, scratch), got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows, k, inter", [(1, 256, 256), (32, 1024, 16640), (20, 1280, 128 * 17)])
+def test_streamed_gate_up(gpu, rows, k, inter):
+    """The SwiGLU pair against the plain projection of the same interleaved weight: its own roundings applied to it."""
+    x, packed, _ = inputs(rows, k, 2 * inter, False)
+    tiles, scales = ext.pack_weight(*packed)
+    from qwen38_amd.steps import act_tiles_to_rows
+
+    got = act_tiles_to_rows(ext.mlp_up(x, rows, k, tiles, scales, inter), 32, inter)[:rows].float()
+    y = ext.fp8_linear(x, tiles, scales, 2 * inter).reshape(rows, inter // 32, 2, 32)
+    gate, up = y[:, :, 0].reshape(rows, inter), y[:, :, 1].reshape(rows, inter)
+    want = round_e5m2(gate * torch.sigmoid(gate) * up).float()
+    # The sums are the same numbers in both, but for tiles split differently (their float32 sums, and so a bf16 rounding,
+    # may fall the other way) and the sigmoid's last bit: an e5m2 step, a quarter of the value at most, at few values.
+    assert float((got != want).float().mean()) <= 2e-3
+    assert bool(((got - want).abs() <= 0.26 * want.abs() + 2.0**-16).all())
