@@ -14,10 +14,10 @@
 // three more launches, so that every (row, KV head) spreads over several workgroups (each kernel skips the rows the
 // other path takes); for them attn_fused only prepares the row once: its query rows normed and rotated (qprep) and
 // the step's own keys, normed and rotated, and values (kv_own).
-//   attn_scores (chunk of 512 cached positions, KV head, row): the prepared query rows, the chunk's scores by MFMA
-//       (sixteen waves, one block of 32 positions each), the chunk's per-row max m_c, the sum s_c of e = exp(s - m_c),
-//       and the scores s themselves (stored as bf16: each is bf16 / 16, so two bytes hold it exactly; rows past the
-//       real query rows are not stored). Chunk 0 also scores the step's own keys.
+//   attn_scores (chunk of 512 cached positions or less, KV head, row; a wave each): the prepared query rows, the chunk's
+//       scores by MFMA, the chunk's per-row max m_c, the sum s_c of e = exp(s - m_c), and the scores s themselves (stored as
+//       bf16: each is bf16 / 16, so two bytes hold it exactly; rows past the real query rows are not stored). Chunk 0
+//       also scores the step's own keys.
 //   attn_pv (split of the row's positions, KV head, row; eight waves, all 256 dims): the row's max M and sum
 //       S = sum_c s_c e^(m_c - M) + own terms; per group of 64 positions, each bf16 weight bf16(e * (e^(m_c - M) / S))
 //       formed once from the stored scores (e = exp(s - m_c), the same float32 values attn_scores summed) into LDS,
@@ -50,7 +50,6 @@
 
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef uint32_t u4t __attribute__((ext_vector_type(4)));
-typedef uint32_t u2t __attribute__((ext_vector_type(2)));
 
 namespace {
 
@@ -457,110 +456,155 @@ __global__ __launch_bounds__(SW * 64) void attn_fused_kernel(const AttnArgs a) {
     }
 }
 
-template <int QT, bool KV8>
-__global__ __launch_bounds__(SW * 64) void attn_scores_kernel(const AttnArgs a) {
-    __shared__ __attribute__((aligned(16))) bf16_t qb[QT * 32 * QPITCH];
-    __shared__ __attribute__((aligned(16))) bf16_t kb[ATTN_KMAX * QPITCH];  // own keys (chunk 0)
-    __shared__ float wred[SW][QT * 32], mrow[QT * 32];
-
-    const int c = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int K = a.K, G = a.Hq / a.Hkv, NQ = G * K, S = a.S;
+// Scores of the chunked path, bound by the key stream from HBM: a wave takes one chunk of a (row, KV head)'s positions by
+// itself, 16 at a time, with the NT * 16 prepared query rows in registers (v_mfma_f32_16x16x32_bf16: A = 16 keys x 32 dims,
+// B = 32 dims x 16 query rows; lane l, g = l / 16, takes dims 64 g + 8 s .. + 7 in step s). The keys go through a ring in LDS
+// that is the wave's own, so there is no barrier: copied a KB of contiguous cache per instruction, read back per lane
+// without bank conflicts (16-byte piece c of row r lies at c ^ r). Each lane carries the maximum and the sum of e^(s - max)
+// over its own positions of its query row; the four lanes of a row merge theirs at the chunk's end.
+// 16 x 4 heads of 28,672 positions on average, 24 query rows: 213 us (0.94 GB of keys, 88 MB of scores, 4.8 TB/s); 64 x 4
+// heads of 7,168, FP8, 6 query rows: 110 us (0.47 GB, 4.3 TB/s). Before, as sixteen waves of 32 positions each around two
+// barriers, 231 and 157 us; with keys read straight into operand registers 251 and 129 us (every load touches 64 cache
+// lines, and the CU's line rate, not HBM, sets the pace); 32 positions at a time, which leaves room for one wave per SIMD,
+// 218 and 135 us; with each block's scores stored at once 235 and 112 us.
+template <int NT, bool KV8>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void attn_scores_kernel(const AttnArgs a) {
+    constexpr int ROW = KV8 ? 256 : 512, BLK = 16 * ROW, NCP = BLK / 1024, RPC = 1024 / ROW;  // bytes; copies per block, rows per copy
+    constexpr int ST = 16384 / BLK;  // ring stages
+    __shared__ __attribute__((aligned(1024))) uint8_t ring[4][ST][BLK];
+    const int kvh = blockIdx.y, b = blockIdx.z, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = blockIdx.x * 4 + wave, r = lane & 15, grp = lane >> 4;
+    const int K = a.K, NQ = a.Hq / a.Hkv * K, S = a.S;
     const int npos = visible(a, b);
     if (npos <= a.fused_max) return;  // attn_fused takes this row
-    const int p_lo = c * ATTN_CHUNK, p_hi = min(p_lo + ATTN_CHUNK, npos);
-    const bool first = c == 0;  // also does the step's own keys
-    if (!first && p_lo >= p_hi) return;
+    const int p_lo = c * a.chunk, p_hi = min(p_lo + a.chunk, npos);
+    if (p_lo >= p_hi) return;
     const size_t head = (size_t)b * a.Hkv + kvh;
-    const int blk = (p_lo >> 5) + wave;  // this wave's 32 positions
-    const bool scored = blk * 32 < p_hi;
+    const int nb = (p_hi - p_lo + 15) >> 4;
 
-    // The query rows as attn_fused prepared them (normed, rotated; chunk 0 also the step's own keys) first, then the
-    // cache keys (clamped into the cache for waves past the chunk's positions, whose scores are never formed), so that
-    // the copy into LDS waits for its own loads only.
-    constexpr int QP = QT * 32 * 32 / (SW * 64);  // 16-byte pieces of the query rows per thread
-    const bf16_t* qsrc = a.qprep + head * ATTN_QMAX * 256;
-    uint4 qv[QP];
+    const uint32_t lds0 = (uint32_t)(uintptr_t)LDS_PTR(&ring[wave][0][0]);
+    const uint8_t* kg = (const uint8_t*)a.k_cache + (head * S + p_lo) * ROW;
+    const int row_in = lane / (64 / RPC), piece = lane % (64 / RPC);  // of one copy: its row, the lane's 16-byte piece
+    auto copy = [&](int n) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < QP; ++u) qv[u] = *(const uint4*)(qsrc + (tid + u * SW * 64) * 8);
-    const float* ksrc = a.kv_own + head * 2 * ATTN_KMAX * 256;
-    float4 kv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // own keys: 4 of K x 256 per thread (chunk 0)
-    if (first && tid * 4 < K * 256) kv = *(const float4*)(ksrc + tid * 4);
-    asm volatile("" ::: "memory");
-    v8bf kf[16];
-    load_keys<KV8>(a, head, min(blk * 32, S - 32), lane, kf);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);  // nor may the copies (and their waits) be scheduled above the key loads
+        for (int j = 0; j < NCP; ++j)
+            lds_quad(kg + (size_t)n * BLK + j * 1024, (uint32_t)(row_in * ROW + ((piece ^ (j * RPC + row_in)) << 4)),
+                     lds0 + (n % ST) * BLK + j * 1024);
+    };
 #pragma unroll
-    for (int u = 0; u < QP; ++u) {
-        const int i = tid + u * SW * 64, r = i >> 5, d = (i & 31) * 8;
-        *(uint4*)(qb + r * QPITCH + d) = qv[u];
+    for (int n = 0; n < ST; ++n)
+        if (n < nb) copy(n);
+    v8bf qf[NT][8];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const bf16_t* qp = a.qprep + (head * ATTN_QMAX + t * 16 + r) * 256 + grp * 64;
+#pragma unroll
+        for (int s = 0; s < 8; ++s) qf[t][s] = load8(qp + s * 8);
     }
-    if (first && tid * 4 < K * 256) {
-        const int t = (tid * 4) >> 8, d = (tid * 4) & 255;
-        *(uint2*)(kb + t * QPITCH + d) = make_uint2(pk_bf16(kv.x, kv.y), pk_bf16(kv.z, kv.w));
-    }
-    __syncthreads();
-
-    // The wave's block of scores, kept in registers; chunk 0's last wave also scores the own keys.
-    v16f sacc[QT];
-    float lmax[QT];
+    constexpr float LOG2E = 1.4426950408889634f;
+    const float ksc = KV8 ? bf2f(*a.k_scale) : 0.0f;
+    float mx[NT], sum[NT];
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt) lmax[qt] = -INFINITY;
-    if (scored) score_block<QT>(kf, qb, lane, blk * 32, p_hi, sacc, lmax);
-    if (first && wave == SW - 1)
-        own_scores<QT>(qb, kb, lane, K, NQ,
-                       [&](int q, int tp, float v) { a.own[(head * ATTN_QMAX + q) * ATTN_KMAX + tp] = v; });
-
+    for (int t = 0; t < NT; ++t) mx[t] = -INFINITY, sum[t] = 0.0f;
+    bf16_t* sr = a.scores + head * ATTN_QMAX * S + p_lo + grp * 4;
+    auto score = [&](int n, uint2 (&w)[NT]) __attribute__((always_inline)) {
+        const uint32_t kl = lds0 + (n % ST) * BLK + r * ROW;
+        auto at = [&](int c16) { return *(const __attribute__((address_space(3))) u4t*)(uintptr_t)(kl + ((c16 ^ r) << 4)); };
+        v4f acc[NT];
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
-        const float m = fmaxf(lmax[qt], __shfl_xor(lmax[qt], 32));
-        if (lane < 32) wred[wave][qt * 32 + lane] = m;
-    }
-    __syncthreads();
-    if (tid < QT * 32) {
-        float m = wred[0][tid];
+        for (int t = 0; t < NT; ++t) acc[t] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+        auto step = [&](int s, v8bf kf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int w = 1; w < SW; ++w) m = fmaxf(m, wred[w][tid]);
-        mrow[tid] = m;
-    }
-    __syncthreads();
-
-    // Phase C: the sums of the chunk's e = exp(s - m_c), and the scores themselves for attn_out, which forms the same
-    // e from them. A score is bf16(acc) / 16 (score_block), so 16 s is a bf16 value and its upper half keeps it whole:
-    // two bytes a score instead of the four of e.
-    float lsum[QT];
-    bf16_t* sr = a.scores + head * ATTN_QMAX * S;
+            for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[t][s], acc[t], 0, 0, 0);
+        };
+        u4t k[KV8 ? 4 : 8];
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
-        lsum[qt] = 0.0f;
-        if (!scored) continue;
-        const int q = qt * 32 + (lane & 31);
-        const float m = mrow[q];
+        for (int i = 0; i < (KV8 ? 4 : 8); ++i) k[i] = at(grp * (KV8 ? 4 : 8) + i);
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const float s[4] = {sacc[qt][g * 4], sacc[qt][g * 4 + 1], sacc[qt][g * 4 + 2], sacc[qt][g * 4 + 3]};
-            lsum[qt] += (expf(s[0] - m) + expf(s[1] - m)) + (expf(s[2] - m) + expf(s[3] - m));
-            uint32_t hi[4];
+        for (int i = 0; i < (KV8 ? 4 : 8); ++i) {
+            if constexpr (KV8) {
+                step(2 * i, __builtin_bit_cast(v8bf, kv_widen8(k[i][0], k[i][1], ksc)));
+                step(2 * i + 1, __builtin_bit_cast(v8bf, kv_widen8(k[i][2], k[i][3], ksc)));
+            } else {
+                step(i, __builtin_bit_cast(v8bf, k[i]));
+            }
+        }
+        const int left = p_hi - p_lo - n * 16 - grp * 4;  // of this lane's four positions, those that are the chunk's
 #pragma unroll
-            for (int i = 0; i < 4; ++i) hi[i] = __float_as_uint(s[i] * 16.0f) >> 16;
-            if (q < NQ)  // rows past NQ are never read
-                *(uint2*)(sr + (size_t)q * S + blk * 32 + g * 8 + (lane >> 5) * 4) =
-                    make_uint2(hi[0] | hi[1] << 16, hi[2] | hi[3] << 16);
+        for (int t = 0; t < NT; ++t) {
+            // A score is bf16(acc) / 16: the bf16 itself is stored, for attn_pv to form the same e^(s - max).
+            w[t] = make_uint2(pk_bf16(acc[t][0], acc[t][1]), pk_bf16(acc[t][2], acc[t][3]));
+            float s[4] = {lo_bf(w[t].x) * 0.0625f, hi_bf(w[t].x) * 0.0625f, lo_bf(w[t].y) * 0.0625f, hi_bf(w[t].y) * 0.0625f};
+            if (n == nb - 1)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) s[i] = i < left ? s[i] : -INFINITY;
+            // From a finite number, so that a lane without a position yet forms no -inf - -inf.
+            const float m = fmaxf(mx[t], fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]))), mf = fmaxf(m, -3.0e38f);
+            float e = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) e += __builtin_amdgcn_exp2f((s[i] - mf) * LOG2E);
+            sum[t] = sum[t] * __builtin_amdgcn_exp2f((mx[t] - mf) * LOG2E) + e;
+            mx[t] = m;
+        }
+    };
+    // Block n has landed when at most the later blocks' copies are outstanding; its stage is refilled once its reads are done.
+    // The scores of four blocks are stored together: whole 128-byte lines of a row at a time (a quarter at a time, lines
+    // leave L2 half written under the key stream), and their completion, which the in-order counter puts before that of
+    // later copies, is waited for once.
+    uint2 w[4][NT];
+    for (int n = 0; n < nb; n += 4) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            if (n + d >= nb) break;
+            if (n + d + ST <= nb)
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"((ST - 1) * NCP) : "memory");
+            else
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            score(n + d, w[d]);
+            if (d == 3 || n + d == nb - 1)
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+                    if (t * 16 + r < NQ)  // rows past NQ are never read
+#pragma unroll
+                        for (int e = 0; e <= d; ++e) *(uint2*)(sr + (size_t)(t * 16 + r) * S + (n + e) * 16) = w[e][t];
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (n + d + ST < nb) copy(n + d + ST);
         }
     }
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
-        const float s = lsum[qt] + __shfl_xor(lsum[qt], 32);
-        if (lane < 32) wred[wave][qt * 32 + lane] = s;
+    for (int t = 0; t < NT; ++t) {
+        float m = fmaxf(mx[t], __shfl_xor(mx[t], 16));
+        m = fmaxf(m, __shfl_xor(m, 32));
+        float e = mx[t] == -INFINITY ? 0.0f : sum[t] * __builtin_amdgcn_exp2f((mx[t] - m) * LOG2E);
+        e += __shfl_xor(e, 16);
+        e += __shfl_xor(e, 32);
+        if (lane < 16)
+            *(float2*)(a.stats + ((head * a.nchunks + c) * ATTN_QMAX + t * 16 + lane) * 2) = make_float2(m, m == -INFINITY ? 0.0f : e);
     }
-    __syncthreads();
-    if (tid < QT * 32) {
-        float s = 0.0f;
+    if (c) return;
+    // The step's own keys: query row q = g K + t sees own tokens t' <= t (rows past K read as zero).
+    v4f acc[NT];
 #pragma unroll
-        for (int w = 0; w < SW; ++w) s += wred[w][tid];
-        float* st = a.stats + ((head * a.nchunks + c) * ATTN_QMAX + tid) * 2;
-        st[0] = mrow[tid];
-        st[1] = mrow[tid] == -INFINITY ? 0.0f : s;
+    for (int t = 0; t < NT; ++t) acc[t] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+    const float* ok = a.kv_own + (head * 2 * ATTN_KMAX + min(r, K - 1)) * 256 + grp * 64;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        const v4f k0 = *(const v4f*)(ok + s * 8), k1 = *(const v4f*)(ok + s * 8 + 4);
+        u4t w = {pk_bf16(k0[0], k0[1]), pk_bf16(k0[2], k0[3]), pk_bf16(k1[0], k1[1]), pk_bf16(k1[2], k1[3])};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = r < K ? w[e] : 0;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, w), qf[t][s], acc[t], 0, 0, 0);
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int q = t * 16 + r;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int tp = grp * 4 + i;
+            if (tp < K && q < NQ) a.own[(head * ATTN_QMAX + q) * ATTN_KMAX + tp] = tp <= q % K ? rbf(acc[t][i]) * 0.0625f : -INFINITY;
+        }
     }
 }
 
@@ -579,7 +623,7 @@ __device__ __forceinline__ void pv_row_stats(const AttnArgs& a, size_t head, int
     constexpr int R = QT * 32, P = 512 / R;
     const int K = a.K, NQ = a.Hq / a.Hkv * K;
     const int r = tid % R, p = tid / R;
-    const int nch = (npos + ATTN_CHUNK - 1) / ATTN_CHUNK, c0 = p * nch / P, c1 = (p + 1) * nch / P;
+    const int nch = (npos + a.chunk - 1) / a.chunk, c0 = p * nch / P, c1 = (p + 1) * nch / P;
     const float* st = a.stats + head * a.nchunks * ATTN_QMAX * 2 + r * 2;
     float m = -INFINITY;
     for (int c = c0; c < c1; ++c) m = fmaxf(m, st[c * ATTN_QMAX * 2]);
@@ -704,15 +748,16 @@ __device__ __forceinline__ void pv_finish(const AttnArgs& a, int b, int kvh, siz
 // bf16(e^(s - m_c) * (e^(m_c - M) / S)) once each, from the scores and chunk maxima attn_scores stored (the float32
 // values it summed), into an LDS tile; wave w multiplies the tile with dims 32w .. 32w + 31 of V by MFMA
 // (A = 32 query rows x 16 positions from LDS, B = 16 positions x 32 dims from registers), adding the groups in
-// position order. Loads run PF groups ahead (slot j of each round of PF; past the range they load the last
+// position order. With up to 16 query rows (decode) only those are formed: forming, with V's widening from FP8, is
+// what the vector units have no time for beside the stream. Loads run PF groups ahead (slot j of each round of PF; past the range they load the last
 // group again, never used, so that every load is unconditional). With one split the workgroup finishes the row;
 // with more, each stores its sums and attn_pv_finish adds them in split order.
-template <int QT, bool KV8>
+template <int QT, bool KV8, int ROWS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void attn_pv_kernel(const AttnArgs a) {
-    constexpr int WPT = QT * 32 * PV_GP / 512;  // weights formed per thread per group (4 or 8)
-    // Groups whose loads a wave keeps in flight: four, or three where two query tiles of bf16 V would not fit
-    // 128 VGPRs (two workgroups per CU) with four.
-    constexpr int PF = QT == 2 && !KV8 ? 3 : 4;
+    constexpr int WPT = ROWS * PV_GP / 512;  // weights formed per thread per group (2, 4 or 8)
+    // Groups whose loads a wave keeps in flight: four, or three where bf16 V would not fit 128 VGPRs (two workgroups
+    // per CU) with four.
+    constexpr int PF = (QT == 2 || ROWS == 16) && !KV8 ? 3 : 4;
     constexpr int NT = PF % 2 == 0 ? 2 : PF;    // LDS weight tiles (slot j writes tile j % NT)
     constexpr int TILE = QT * 32 * PV_WP;       // bf16 per LDS weight tile
     constexpr int SMEM = NT * TILE * 2 > 32 * PV_RP * 4 ? NT * TILE * 2 : 32 * PV_RP * 4;
@@ -737,7 +782,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void a
     // Slot loads: V of this wave's dims over the group's 64 positions (lane half h: positions 16 kk + 8 h .. + 7 of
     // MFMA step kk), the scores of the weights this thread forms and their chunk's max.
     typedef typename std::conditional<KV8, uint2, v8bf>::type VSlot;
-    typedef typename std::conditional<WPT == 8, u4t, u2t>::type SSlot;
+    typedef uint32_t SSlot __attribute__((ext_vector_type(WPT / 2)));
     VSlot vs[PF][4];
     SSlot ss[PF];
     float mc[PF];
@@ -752,7 +797,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void a
                 vs[j][kk] = load8(a.v_cache + vo);
         }
         ss[j] = *(const SSlot*)(sr + (size_t)lr * S + min(g * PV_GP + fc, S - WPT));
-        mc[j] = cst[((g * PV_GP / ATTN_CHUNK) * ATTN_QMAX + lr) * 2];
+        mc[j] = cst[((g * PV_GP / a.chunk) * ATTN_QMAX + lr) * 2];
     };
 #pragma unroll
     for (int j = 0; j < PF; ++j) issue(j, g_lo + j);
@@ -770,20 +815,24 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void a
     // Group g from slot j: its weights into tile w (positions at or past npos, and rows past NQ, weigh zero).
     const int nlim = fr < NQ ? npos : 0;
     auto form = [&](int j, int g, bf16_t* w) {
-        const float m = mc[j], f = expf(m - fm) * fi;
+        constexpr float LOG2E = 1.4426950408889634f;
+        const float m = mc[j], f = __builtin_amdgcn_exp2f((m - fm) * LOG2E) * fi;
         const int p0 = g * PV_GP + fc;
-        uint32_t words[WPT / 2];
+        SSlot words;
 #pragma unroll
         for (int e = 0; e < WPT / 2; ++e) {
             const uint32_t pair = ss[j][e];
-            const float s0 = bf2f(pair & 0xffff) * 0.0625f, s1 = bf2f(pair >> 16) * 0.0625f;
-            words[e] = pk_bf16(p0 + 2 * e < nlim ? expf(s0 - m) * f : 0.0f, p0 + 2 * e + 1 < nlim ? expf(s1 - m) * f : 0.0f);
+            const float e0 = __builtin_amdgcn_exp2f((lo_bf(pair) * 0.0625f - m) * LOG2E) * f;
+            const float e1 = __builtin_amdgcn_exp2f((hi_bf(pair) * 0.0625f - m) * LOG2E) * f;
+            words[e] = pk_bf16(p0 + 2 * e < nlim ? e0 : 0.0f, p0 + 2 * e + 1 < nlim ? e1 : 0.0f);
         }
-        if constexpr (WPT == 8)
-            *(uint4*)(w + fr * PV_WP + fc) = make_uint4(words[0], words[1], words[2], words[3]);
-        else
-            *(uint2*)(w + fr * PV_WP + fc) = make_uint2(words[0], words[1]);
+        *(SSlot*)(w + fr * PV_WP + fc) = words;
     };
+    if constexpr (ROWS < QT * 32)  // the tiles' other rows weigh nothing, once and for all
+        for (int i = tid; i < NT * (QT * 32 - ROWS) * PV_WP / 2; i += 512) {
+            constexpr int PER = (QT * 32 - ROWS) * PV_WP / 2;
+            ((uint32_t*)wt)[(i / PER) * (TILE / 2) + ROWS * PV_WP / 2 + i % PER] = 0;
+        }
     auto mfma = [&](int j, const bf16_t* w) {
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
@@ -881,8 +930,21 @@ hipError_t launch_attn(AttnArgs a, hipStream_t stream) {
         int ns = pairs >= 2L * a.cus ? 1 : (int)std::min<long>(PV_SPLIT_MAX, std::max<long>(1, 2L * a.cus / pairs));
         while (ns > 1 && (size_t)pairs * ns * QT * 8192 > a.pv_part_floats) --ns;
         a.pv_splits = ns;
-        hipLaunchKernelGGL((attn_scores_kernel<QT, KV8>), dim3(a.nchunks, a.Hkv, a.B), dim3(SW * 64), 0, stream, a);
-        hipLaunchKernelGGL((attn_pv_kernel<QT, KV8>), dim3(ns, pairs), dim3(512), 0, stream, a);
+        // Positions per wave of attn_scores: 512, fewer while that leaves less than three rounds of the eight waves a CU
+        // holds (over the whole cache: the rows' own lengths are on the device), so that the last round is a short one:
+        // scores and weights x V 202 + 117 us with 256 against 221 + 117 with 512 at the shapes above.
+        a.chunk = ATTN_CHUNK;
+        while (a.chunk > ATTN_CHUNK_MIN && pairs * ((a.S + a.chunk - 1) / a.chunk) < 24L * a.cus) a.chunk /= 2;
+        a.nchunks = (a.S + a.chunk - 1) / a.chunk;
+        const dim3 grid((a.nchunks + 3) / 4, a.Hkv, a.B);
+        if (a.Hq / a.Hkv * a.K <= 16)
+            hipLaunchKernelGGL((attn_scores_kernel<1, KV8>), grid, dim3(256), 0, stream, a);
+        else
+            hipLaunchKernelGGL((attn_scores_kernel<2 * QT, KV8>), grid, dim3(256), 0, stream, a);
+        if (QT == 1 && a.Hq / a.Hkv * a.K <= 16)
+            hipLaunchKernelGGL((attn_pv_kernel<1, KV8, 16>), dim3(ns, pairs), dim3(512), 0, stream, a);
+        else
+            hipLaunchKernelGGL((attn_pv_kernel<QT, KV8, QT * 32>), dim3(ns, pairs), dim3(512), 0, stream, a);
         if (ns > 1) hipLaunchKernelGGL((attn_pv_finish_kernel<QT, KV8>), dim3(4, pairs), dim3(128), 0, stream, a);
     }
     return hipGetLastError();
@@ -892,7 +954,7 @@ hipError_t launch_attn(AttnArgs a, hipStream_t stream) {
 
 hipError_t q38_attn_verify(const AttnArgs& a, hipStream_t stream) {
     const int NQ = a.Hq / a.Hkv * a.K;
-    if (NQ > ATTN_QMAX || a.K > ATTN_KMAX || (long)a.nchunks * ATTN_CHUNK < a.S) return hipErrorInvalidValue;
+    if (NQ > ATTN_QMAX || a.K > ATTN_KMAX || (long)a.nchunks * ATTN_CHUNK_MIN < a.S) return hipErrorInvalidValue;
     if (a.S < 32 || a.S % 32) return hipErrorInvalidValue;  // whole blocks of 32 positions (every wave loads one)
     // Two position blocks per wave need 66 KB of bf16 weights in LDS at 32 query rows; 64 rows keep one.
     if (a.kv8) {

@@ -31,6 +31,14 @@ typedef __bf16 v8bf16 __attribute__((ext_vector_type(8)));
 // A __shared__ object as an LDS address (its 32-bit value is the LDS byte offset the direct global -> LDS copies take).
 #define LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
 
+// Direct global -> LDS copy of 16 bytes per lane from base + off (base wave-uniform, in scalar registers): lane l's bytes
+// land at LDS address dst + 16 l (dst wave-uniform). Inline assembly, so the compiler neither counts it nor waits for it;
+// the kernels' own vmcnt waits cover it.
+__device__ __forceinline__ void lds_quad(const void* base, uint32_t off, uint32_t dst) {
+    const uint32_t m0 = __builtin_amdgcn_readfirstlane(dst);
+    asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(m0) : "memory");
+}
+
 __device__ __forceinline__ float bf2f(bf16_t h) { return __uint_as_float(((uint32_t)h) << 16); }
 
 // The bf16 in the low / high half of a word, widened.

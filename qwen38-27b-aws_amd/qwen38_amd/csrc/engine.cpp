@@ -97,7 +97,7 @@ struct q38_handle {
            off_prows = 0, off_pkw = 0, off_pvw = 0;
     size_t part_floats;  // capacity of the split-K partial buffer
     int gate_groups;  // K ranges of the gated-delta gate projections
-    int attn_nchunks;  // chunks of ATTN_CHUNK cached positions over S
+    int attn_nchunks;  // chunks of ATTN_CHUNK_MIN cached positions over S
     size_t prefill_slots = 0;  // slots of the prefill attention's partial sums
     size_t attn_pv_floats;  // capacity of the chunked attention's split sums
     // Kernel timer (q38_kernel_timer): event pairs around the gate/up GEMM launches while on.
@@ -709,14 +709,14 @@ int q38_create(const q38_config* cfg, q38_handle** out) {
     while (h->gate_groups > 1 && (h->H % (64 * h->gate_groups) || h->H / (64 * h->gate_groups) > 16)) h->gate_groups /= 2;
     h->off_gates = take((size_t)h->gate_groups * Tp * 2 * h->Hv * 4);
     const size_t heads = (size_t)h->B * h->Hkv;
-    h->attn_nchunks = (h->S + ATTN_CHUNK - 1) / ATTN_CHUNK;
+    h->attn_nchunks = (h->S + ATTN_CHUNK_MIN - 1) / ATTN_CHUNK_MIN;
     h->off_scores = take(heads * ATTN_QMAX * h->S * 2);
     h->off_astats = take(heads * h->attn_nchunks * ATTN_QMAX * 2 * 4);
     h->off_aown = take(heads * ATTN_QMAX * ATTN_KMAX * 4);
     h->off_akv = take(heads * 2 * ATTN_KMAX * 256 * 4);
     h->off_aq = take(heads * ATTN_QMAX * 256 * 2);
     // attn_pv's split sums: at most about two workgroups per CU of 64 query rows x 256 dims each.
-    h->attn_pv_floats = h->attn_nchunks > 1 ? (size_t)2 * device_cus() * ATTN_QMAX * 256 : 0;
+    h->attn_pv_floats = h->S > ATTN_CHUNK ? (size_t)2 * device_cus() * ATTN_QMAX * 256 : 0;
     h->off_apv = take(h->attn_pv_floats * 4);
     h->off_apr = take(heads * ATTN_QMAX * (2 + ATTN_KMAX) * 4);
     h->off_htiles = take(Tv * H * 2);

@@ -161,7 +161,8 @@ inline size_t prefill_slots(int L, int Hq, int Hkv) {
 
 #define ATTN_KMAX 8   // verify tokens
 #define ATTN_QMAX 64  // query rows per KV head
-#define ATTN_CHUNK 512  // cached positions per attn_scores workgroup (32 per wave)
+#define ATTN_CHUNK 512  // cached positions of one attn_fused pass (32 per wave), and at most of an attn_scores wave
+#define ATTN_CHUNK_MIN 128  // and at least (a multiple of attn_pv's groups of 64)
 
 struct AttnArgs {
     int B, K, Hq, Hkv, S;
@@ -175,7 +176,8 @@ struct AttnArgs {
     const float* active;
     bf16_t* k_cache;
     bf16_t* v_cache;
-    int nchunks;            // chunks of ATTN_CHUNK cached positions over S
+    int nchunks;            // chunks of `chunk` cached positions over S (from the caller: those of ATTN_CHUNK_MIN, the stats' room)
+    int chunk;              // set by the launcher
     bf16_t* scores;         // [B*Hkv][ATTN_QMAX][S]: the scores times 16 (bf16-exact); attn_pv forms exp(s - chunk max)
     float* stats;           // [B*Hkv][nchunks][ATTN_QMAX][2]: per chunk, max and sum of exp(score - max)
     float* own;             // [B*Hkv][ATTN_QMAX][ATTN_KMAX]: scores of the step's own keys (-inf where masked)

@@ -39,14 +39,6 @@ __device__ __forceinline__ float conv_window(const PrefillGdnArgs& a, const bf16
 
 __device__ __forceinline__ v4f mfma16(float x, float y, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0); }
 
-// Direct global -> LDS copy of 16 bytes per lane from base + off (base wave-uniform, in scalar registers): lane l's bytes
-// land at LDS address dst + 16 l (dst wave-uniform). Inline assembly, so the compiler neither counts it nor waits for it;
-// the kernels' own vmcnt waits cover it.
-__device__ __forceinline__ void lds_quad(const void* base, uint32_t off, uint32_t dst) {
-    const uint32_t m0 = __builtin_amdgcn_readfirstlane(dst);
-    asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(m0) : "memory");
-}
-
 // e^x of a 64-bit x, in float32 without x's own rounding (|x| ulps of the result).
 __device__ __forceinline__ float exp_of(double x) {
     const float hi = (float)x, e = expf(hi);
