@@ -45,6 +45,16 @@ __device__ __forceinline__ float bf2f(bf16_t h) { return __uint_as_float(((uint3
 __device__ __forceinline__ float lo_bf(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float hi_bf(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 
+// 8 E2M1 weights (one word, the first input in the lowest nibble) times 2^(scale byte - 127) as one bf16 MFMA operand.
+__device__ __forceinline__ v8bf16 widen_e2m1(uint32_t w, float scale) {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    u4 r = {__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 0)),
+            __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 1)),
+            __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 2)),
+            __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 3))};
+    return __builtin_bit_cast(v8bf16, r);
+}
+
 // fp32 -> bf16, round to nearest even (c10::BFloat16's rounding; v_cvt_pk_bf16_f32); NaN stays NaN.
 __device__ __forceinline__ bf16_t f2bf(float f) { return __builtin_bit_cast(bf16_t, (__bf16)f); }
 

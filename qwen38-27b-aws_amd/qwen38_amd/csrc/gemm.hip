@@ -107,15 +107,6 @@ __device__ __forceinline__ v8bf widen_e5m2(uint32_t x0, uint32_t x1) {
     return __builtin_bit_cast(v8bf, r);
 }
 
-// 8 E2M1 weights (one word, the first input in the lowest nibble) times 2^(scale byte - 127) as one bf16 MFMA operand.
-__device__ __forceinline__ v8bf widen_e2m1(uint32_t w, float scale) {
-    u4 r = {bits(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 0)),
-            bits(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 1)),
-            bits(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 2)),
-            bits(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 3))};
-    return __builtin_bit_cast(v8bf, r);
-}
-
 template <int WF, int WT, int FR, int TR, bool A8, int S, int EPI, bool W4, bool F8, int KU>
 __global__ __launch_bounds__(WF * WT * 64, 1) void gemm_kernel(const GemmArgs a) {
     constexpr int NW = WF * WT, NTH = NW * 64;
@@ -384,13 +375,6 @@ __global__ __launch_bounds__(WF * WT * 64, 1) void gemm_kernel(const GemmArgs a)
                         bf16_t* dst = col < a.n0 ? (bf16_t*)a.out0 + (size_t)tok * a.ld0 + col
                                                  : (bf16_t*)a.out1 + (size_t)tok * a.ld1 + (col - a.n0);
                         float v[4] = {acc[f][t][g * 4 + 0], acc[f][t][g * 4 + 1], acc[f][t][g * 4 + 2], acc[f][t][g * 4 + 3]};
-                        if (a.accumulate) {  // bf16(out + bf16(sum)), the reference's sum of two bf16 products
-                            const uint2 old = *(const uint2*)dst;
-                            v[0] = lo_bf(old.x) + rbf(v[0]);
-                            v[1] = hi_bf(old.x) + rbf(v[1]);
-                            v[2] = lo_bf(old.y) + rbf(v[2]);
-                            v[3] = hi_bf(old.y) + rbf(v[3]);
-                        }
                         *(uint2*)dst = make_uint2(pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3]));
                     }
                 }
@@ -1011,11 +995,6 @@ hipError_t dispatch(const GemmArgs& a, int* splits_out, hipStream_t stream) {
 }  // namespace
 
 hipError_t q38_gemm(const GemmArgs& a, int epi, int* splits_out, hipStream_t stream) {
-    if (a.w4 && a.bf16_act) {
-        // bf16 activation tiles against MXFP4 weights (the reference's FP4Linear numerics, one plane per launch)
-        if (epi != EPI_BF16) return hipErrorInvalidValue;
-        return dispatch<false, EPI_BF16, true, false>(a, splits_out, stream);
-    }
     if (a.w4) {
         switch (epi) {
             case EPI_BF16: return dispatch<true, EPI_BF16, true, false>(a, splits_out, stream);
