@@ -620,8 +620,9 @@ __global__ __launch_bounds__(WF * WT * 64, 1) void gemm_kernel(const GemmArgs a)
     }
 }
 
-// Up to 64 tokens: a weight-streaming kernel, bound by HBM. A workgroup of KW waves works on 64 features; its waves split
-// the K range and each takes all tokens, so nothing is shared between waves before a tile's end: weights, scales and
+// Up to 128 tokens: a weight-streaming kernel, bound by HBM. A workgroup of KW waves works on 64 features; its waves split
+// the K range and each takes all tokens (bf16 outputs from 65 tokens up: a block of 64, whose sums leave registers for the
+// loads), so nothing is shared between waves before a tile's end: weights, scales and
 // activations go straight to registers, D K-steps ahead (a K-step is 4 KiB of e4m3 weights per wave), with no ring and no
 // barrier; at the end the waves' sums are added in K order through LDS, one feature tile at a time, with the next tile's
 // first loads in flight. (With 128 to 512 features per workgroup in the ring kernel, a tile's K range was split over up
@@ -634,17 +635,20 @@ __global__ __launch_bounds__(WF * WT * 64, 1) void gemm_kernel(const GemmArgs a)
 template <int TT, int EPI, bool W4, int KW>
 __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(2))) void gemm_stream_kernel(const GemmArgs a) {
     constexpr int FR = 2, WTB = W4 ? 1024 : 2048;
-    constexpr int D = TT == 1 ? 4 : 3;  // K-steps in flight
+    constexpr int D = TT == 1 ? 4 : TT == 2 ? 3 : 2;  // K-steps in flight
     static_assert(D * (5 * FR + 4 * TT) <= 63, "vmcnt range");
     constexpr int G = TT * 4, GW = (G + KW - 1) / KW;  // (token tile, quarter of the rows) quads of a feature tile, per wave
     __shared__ __attribute__((aligned(16))) float red[KW * G * 256];
     __shared__ unsigned long long s_arrived;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int tiles = a.N / (32 * FR), KS = a.K >> 6;
+    const int blocks = a.Tpad / (32 * TT), tiles = a.N / (32 * FR) * blocks, KS = a.K >> 6;
 
     struct Seg {
-        int fb, k0, k1;  // K-steps [k0, k1) of tile fb
+        int tile, k0, k1;  // K-steps [k0, k1) of a tile
     };
+    // A tile's 64 features and its block of tokens: a feature tile's blocks 8 ids apart, on one XCD, where the counts allow.
+    auto fb_of = [&](int tile) { return tiles % (8 * blocks) ? tile / blocks : tile / (8 * blocks) * 8 + tile % 8; };
+    auto tb_of = [&](int tile) { return tiles % (8 * blocks) ? tile % blocks : tile / 8 % blocks; };
     typedef typename std::conditional<W4, uint32_t, u2>::type WFrag;
     struct Step {
         WFrag w[FR][4];
@@ -654,11 +658,11 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     Step st[D];
     // This wave's part of a segment's K range.
     auto part0 = [&](const Seg& s, int w) { return s.k0 + (int)((long)w * (s.k1 - s.k0) / KW); };
-    auto load = [&](int fb, int k, Step& s) __attribute__((always_inline)) {
+    auto load = [&](int fb, int tb, int k, Step& s) __attribute__((always_inline)) {
         k = min(k, KS - 1);  // past the range: loaded, never used
         const uint8_t* wp = a.w + ((size_t)(fb * FR) * KS + k) * WTB;
         const uint8_t* sp = a.ws + ((size_t)(fb * FR) * KS + k) * 64;
-        const uint8_t* xp = (const uint8_t*)a.act + (size_t)k * 2048;
+        const uint8_t* xp = (const uint8_t*)a.act + ((size_t)(tb * TT) * KS + k) * 2048;
 #pragma unroll
         for (int f = 0; f < FR; ++f) {
             s.sc[f] = *(const uint16_t*)(sp + (size_t)f * KS * 64 + (lane & 31) * 2);
@@ -698,9 +702,9 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
         }
     };
     auto fill = [&](const Seg& s) __attribute__((always_inline)) {
-        const int k = part0(s, wave);
+        const int k = part0(s, wave), fb = fb_of(s.tile), tb = tb_of(s.tile);
 #pragma unroll
-        for (int d = 0; d < D; ++d) load(s.fb, k + d, st[d]);
+        for (int d = 0; d < D; ++d) load(fb, tb, k + d, st[d]);
     };
     // The segment's products over this wave's K range, its first D K-steps already on their way.
     auto run = [&](const Seg& s) __attribute__((always_inline)) {
@@ -711,12 +715,12 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
 #pragma unroll
                 for (int i = 0; i < 16; ++i) acc[f][t][i] = 0.0f;
         int k = part0(s, wave);
-        const int k1 = part0(s, wave + 1);
+        const int k1 = part0(s, wave + 1), fb = fb_of(s.tile), tb = tb_of(s.tile);
         for (; k + D <= k1; k += D) {
 #pragma unroll
             for (int d = 0; d < D; ++d) {
                 compute(st[d]);
-                load(s.fb, k + D + d, st[d]);
+                load(fb, tb, k + D + d, st[d]);
             }
         }
 #pragma unroll
@@ -752,12 +756,13 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
             }
         }
     };
-    auto epilogue = [&](int fb, int z) __attribute__((always_inline)) {
+    auto epilogue = [&](int tile, int z) __attribute__((always_inline)) {
+        const int fb = fb_of(tile), tb = tb_of(tile);
 #pragma unroll
         for (int j = 0; j < GW; ++j) {
             const int g = wave + j * KW;
             if (g >= G) break;
-            const int tok = (g >> 2) * 32 + (lane & 31), row = (g & 3) * 8 + (lane >> 5) * 4;
+            const int tok = (tb * TT + (g >> 2)) * 32 + (lane & 31), row = (g & 3) * 8 + (lane >> 5) * 4;
             if constexpr (EPI == EPI_SWIGLU) {
                 float h[4];  // the two feature tiles: gate and up of the same 32 inner features
 #pragma unroll
@@ -789,13 +794,13 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
         fill(s);
         run(s);
         reduce();
-        epilogue(s.fb, z);
+        epilogue(s.tile, z);
     } else {
         const int whole = tiles / a.cus * a.cus, i = (int)blockIdx.x - whole, n = i < 0 ? 1 : a.splits;
         const int rest = (i >> 3) / n * 8 + (i & 7), z = (i >> 3) % n;  // among the split tiles, a tile's parts 8 ids apart
-        const int fb = i < 0 ? (int)blockIdx.x : whole + rest;
-        if (fb >= tiles) return;
-        auto part_of = [&](int p) { return Seg{fb, p * KS / n, (p + 1) * KS / n}; };
+        const int tile = i < 0 ? (int)blockIdx.x : whole + rest;
+        if (tile >= tiles) return;
+        auto part_of = [&](int p) { return Seg{tile, p * KS / n, (p + 1) * KS / n}; };
         const Seg s = part_of(i < 0 ? 0 : z);
         fill(s);
         run(s);
@@ -850,7 +855,7 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
                 for (int j = 0; j < GW; ++j) sum[f][j] = total[f][j];
             if (tid == 0) __hip_atomic_store(a.counters + rest, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        epilogue(fb, 0);
+        epilogue(tile, 0);
     }
 }
 
@@ -860,7 +865,7 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
 template <int TT, int EPI, bool W4, int KW>
 hipError_t launch_stream(const GemmArgs& a0, int* splits_out, hipStream_t stream) {
     GemmArgs a = a0;
-    const int tiles = a.N / 64, KS = a.K / 64, whole = EPI == EPI_PARTIAL ? 0 : tiles / a.cus * a.cus, rest = tiles - whole;
+    const int tiles = a.N / 64 * (a.Tpad / (32 * TT)), KS = a.K / 64, whole = EPI == EPI_PARTIAL ? 0 : tiles / a.cus * a.cus, rest = tiles - whole;
     int s = std::min(std::min(rest ? a.cus / rest : 1, GEMM_SPLIT_MAX), KS / (2 * KW));
     if (EPI == EPI_PARTIAL && a.splits_max > 0) s = std::min(s, a.splits_max);
     a.splits = s = std::max(s, 1);
@@ -873,9 +878,9 @@ hipError_t launch_stream(const GemmArgs& a0, int* splits_out, hipStream_t stream
 
 template <int TT, int EPI, bool W4>
 hipError_t dispatch_stream(const GemmArgs& a, int* splits_out, hipStream_t stream) {
-    if (a.N % 64 || a.K % 64 || a.Tpad != 32 * TT || a.cus < 8 || a.cus % 8) return hipErrorInvalidValue;
+    if (a.N % 64 || a.K % 64 || a.Tpad % (32 * TT) || a.cus < 8 || a.cus % 8) return hipErrorInvalidValue;
     if constexpr (EPI != EPI_PARTIAL)
-        if (a.N / 64 >= 2 * a.cus) return launch_stream<TT, EPI, W4, 4>(a, splits_out, stream);
+        if (a.N / 64 * (a.Tpad / (32 * TT)) >= 2 * a.cus) return launch_stream<TT, EPI, W4, 4>(a, splits_out, stream);
     return launch_stream<TT, EPI, W4, 8>(a, splits_out, stream);
 }
 
@@ -950,16 +955,23 @@ hipError_t dispatch(const GemmArgs& a, int* splits_out, hipStream_t stream) {
             return launch<4, 2, 2, 4, false, 3, EPI, W4, F8>(a, splits_out, stream);
         }
     }
-    // e5m2 activations up to 64 tokens stream their weights, but for the SwiGLU pair at 33 to 64 tokens: there the
+    // e5m2 activations up to 128 tokens stream their weights, but for the SwiGLU pair from 33 tokens up: there the
     // activations that every wave reads for itself weigh as much as the weights (gate/up of the 27B MLP 57 against 48.6 us
     // e4m3, 49 against 42.7 us MXFP4; the bf16 outputs 23 against 28 and 17 against 26 us, the split-K partials 40 against
-    // 48.6 and 30 against 47 us; up to 32 tokens gate/up 42.7 against 45, bf16 outputs 19 against 35, partials 33 against 50).
+    // 48.6 and 30 against 47 us; up to 32 tokens gate/up 42.7 against 45, bf16 outputs 19 against 35, partials 33 against 50). At 65 to 128 tokens the
+    // ring's 512-feature tiles left ten of them to 256 CUs: 100 rows of 5120 -> 14336 43.3 against 58.2 us (as one block of 128
+    // 38.2, but its sums spill), 6144 -> 5120 26.9 against 66.8 us; MXFP4 17408 -> 5120 43.1 against 116.7. Partials take all
+    // 128 tokens: their weights are read once, and split in K they fill the CUs (the 27B layers of 128 tokens 232 against
+    // 245 us with blocks of 64, 284 with the ring).
     constexpr bool RING32 = !A8 || F8, RING64 = RING32 || EPI == EPI_SWIGLU;
     const bool wide = a.N % 512 == 0 && (balanced(512) || !balanced(256));
     switch (a.Tpad) {
         case 128:
-            return wide ? launch<8, 1, 2, 4, A8, 3, EPI, W4, F8>(a, splits_out, stream)
-                        : launch<4, 2, 2, 2, A8, 3, EPI, W4, F8>(a, splits_out, stream);
+            if constexpr (!RING64)
+                return dispatch_stream<EPI == EPI_PARTIAL ? 4 : 2, EPI, W4>(a, splits_out, stream);
+            else
+                return wide ? launch<8, 1, 2, 4, A8, 3, EPI, W4, F8>(a, splits_out, stream)
+                            : launch<4, 2, 2, 2, A8, 3, EPI, W4, F8>(a, splits_out, stream);
         case 64:
             if constexpr (RING64) {
                 // The FP8 MFMA's bf16 outputs as 128 x 64 tiles with a deep ring, its partials with 5 stages; the SwiGLU

@@ -1,4 +1,4 @@
-"""The weight-streaming projection (up to 64 tokens) where its schedule can go wrong: K ranges shorter than a workgroup's
+"""The weight-streaming projection (up to 128 tokens) where its schedule can go wrong: K ranges shorter than a workgroup's
 waves, tiles left over beyond a multiple of the CUs split in K, four-wave workgroups, ragged tokens; e4m3 and MXFP4.
 
 Held against float64: half a bf16 ulp of the result for its rounding, plus 2^-20 of sum |x w| for the float32 sums (as the
@@ -42,6 +42,10 @@ def check(got, x, wd):
         (64, 512, 16640),
         (17, 320 * 4, 33280),  # 520 tiles: four-wave workgroups, 8 left over
         (61, 17408, 5120),  # 80 tiles split 3 ways
+        (65, 256, 256),  # two blocks of 64 tokens
+        (100, 1280, 16640),  # 520 tiles, not eight of a block at a time: four-wave workgroups, 8 left over
+        (128, 17408, 5120),
+        (97, 5120, 4864),  # 152 tiles
     ],
 )
 def test_streamed_projection(gpu, rows, k, n, mx):
@@ -75,3 +79,41 @@ def test_streamed_gate_up(gpu, rows, k, inter):
     # may fall the other way) and the sigmoid's last bit: an e5m2 step, a quarter of the value at most, at few values.
     assert float((got != want).float().mean()) <= 2e-3
     assert bool(((got - want).abs() <= 0.26 * want.abs() + 2.0**-16).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k, n", [(256, 256), (3072, 1024), (5120, 4352)])
+def test_streamed_sums_of_128_tokens(gpu, k, n):
+    """The float32 sums (the split-K form's, one part): 2^-20 of sum |x w|."""
+    x, packed, wd = inputs(128, k, n, False)
+    xq = round_e5m2(x).double()
+    off = (ext.fp8_linear_f32(x, *ext.pack_weight(*packed), n).double() - xq @ wd.T).abs()
+    assert bool((off <= (xq.abs() @ wd.abs().T) * 2.0**-20).all())
+
+
+@pytest.mark.gpu
+def test_streamed_parts_of_96_tokens_match_the_oracle(gpu):
+    """The MTP step of 24 rows x 4 tokens, whose projections are summed from several workgroups' parts: per row within the
+    2e-2 that the step's one layer is held to."""
+    from oracle import model as om
+    from qwen38_amd import synth
+    from qwen38_amd.config import tiny_config
+    from qwen38_amd.generate import mtp_step_inputs
+    from qwen38_amd.steps import Engine, MTPStep
+    from scenario import oracle_weights
+
+    cfg, b, k, s, seed = tiny_config(1), 24, 4, 128, 29
+    context = [(7 * r) % 120 for r in range(b)]
+    values = dict((sp.name, v) for sp, v in synth.make_all(synth.model_specs(cfg), seed))
+    engine = Engine(cfg, b, k, s, mtp=True)
+    engine.load(values.items())
+    mst = synth.kv_states(cfg, b, s, context, seed, "mtp")
+    engine.set_kv(engine.mtp_layer, mst["k_cache"], mst["v_cache"])
+    mi = mtp_step_inputs(cfg, context, k, s, torch.bfloat16, [True] * b)
+    mi["position"] = torch.as_tensor(context, dtype=torch.int32)
+    hidden = synth.hidden_states((b, k, cfg.hidden_size), seed, "stream.hidden")
+    embeds = values["embed_tokens"][torch.randint(0, cfg.vocab_size, (b, k), generator=torch.Generator().manual_seed(seed))]
+    out = MTPStep(engine)(hidden=hidden, inputs_embeds=embeds, **mi).cpu().float().flatten(1)
+    want = om.mtp_forward(cfg, oracle_weights(values, cfg)[1], mst, hidden, embeds, mi["cos"], mi["sin"], mi["position"], mi["active"])
+    want = want.float().flatten(1)
+    assert float(((out - want).norm(dim=1) / want.norm(dim=1)).max()) <= 2e-2
