@@ -632,7 +632,7 @@ __global__ __launch_bounds__(WF * WT * 64, 1) void gemm_kernel(const GemmArgs a)
 // the CUs are one workgroup's each; the rest are split in K over `splits` workgroups on one XCD each, as many as the CUs
 // take, finished by the last to arrive from the others' sums in that XCD's L2 (or, should one have run elsewhere, by
 // computing theirs again). EPI_PARTIAL: K split over workgroups, a part each.
-template <int TT, int EPI, bool W4, int KW>
+template <int TT, int NB, int EPI, bool W4, int KW>  // NB blocks of 32 TT tokens: a constant, as its divisions are 1 to 2 us
 __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(2))) void gemm_stream_kernel(const GemmArgs a) {
     constexpr int FR = 2, WTB = W4 ? 1024 : 2048;
     constexpr int D = TT == 1 ? 4 : TT == 2 ? 3 : 2;  // K-steps in flight
@@ -641,14 +641,14 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     __shared__ __attribute__((aligned(16))) float red[KW * G * 256];
     __shared__ unsigned long long s_arrived;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int blocks = a.Tpad / (32 * TT), tiles = a.N / (32 * FR) * blocks, KS = a.K >> 6;
+    const int tiles = a.N / (32 * FR) * NB, KS = a.K >> 6;
 
     struct Seg {
         int tile, k0, k1;  // K-steps [k0, k1) of a tile
     };
     // A tile's 64 features and its block of tokens: a feature tile's blocks 8 ids apart, on one XCD, where the counts allow.
-    auto fb_of = [&](int tile) { return tiles % (8 * blocks) ? tile / blocks : tile / (8 * blocks) * 8 + tile % 8; };
-    auto tb_of = [&](int tile) { return tiles % (8 * blocks) ? tile % blocks : tile / 8 % blocks; };
+    auto fb_of = [&](int tile) { return NB == 1 ? tile : tiles % (8 * NB) ? tile / NB : tile / (8 * NB) * 8 + tile % 8; };
+    auto tb_of = [&](int tile) { return NB == 1 ? 0 : tiles % (8 * NB) ? tile % NB : tile / 8 % NB; };
     typedef typename std::conditional<W4, uint32_t, u2>::type WFrag;
     struct Step {
         WFrag w[FR][4];
@@ -862,26 +862,26 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
 // Waves per workgroup: eight, one workgroup per CU; four from two tiles per CU up, whose workgroups then share the CUs.
 // Splits: as many as the CUs take (of all tiles with EPI_PARTIAL, else of those beyond a multiple of the CUs), of at least
 // two K-steps per wave.
-template <int TT, int EPI, bool W4, int KW>
+template <int TT, int NB, int EPI, bool W4, int KW>
 hipError_t launch_stream(const GemmArgs& a0, int* splits_out, hipStream_t stream) {
     GemmArgs a = a0;
-    const int tiles = a.N / 64 * (a.Tpad / (32 * TT)), KS = a.K / 64, whole = EPI == EPI_PARTIAL ? 0 : tiles / a.cus * a.cus, rest = tiles - whole;
+    const int tiles = a.N / 64 * NB, KS = a.K / 64, whole = EPI == EPI_PARTIAL ? 0 : tiles / a.cus * a.cus, rest = tiles - whole;
     int s = std::min(std::min(rest ? a.cus / rest : 1, GEMM_SPLIT_MAX), KS / (2 * KW));
     if (EPI == EPI_PARTIAL && a.splits_max > 0) s = std::min(s, a.splits_max);
     a.splits = s = std::max(s, 1);
     const int grid = EPI == EPI_PARTIAL ? tiles * s : whole + (rest + 7) / 8 * 8 * s;
     if (EPI != EPI_PARTIAL && s > 1 && (rest > a.counters_n || (size_t)rest * s * 2 * TT * 1024 > a.fix_floats)) return hipErrorInvalidValue;
     if (splits_out) *splits_out = EPI == EPI_PARTIAL ? s : 1;
-    hipLaunchKernelGGL((gemm_stream_kernel<TT, EPI, W4, KW>), dim3(grid), dim3(KW * 64), 0, stream, a);
+    hipLaunchKernelGGL((gemm_stream_kernel<TT, NB, EPI, W4, KW>), dim3(grid), dim3(KW * 64), 0, stream, a);
     return hipGetLastError();
 }
 
-template <int TT, int EPI, bool W4>
+template <int TT, int NB, int EPI, bool W4>
 hipError_t dispatch_stream(const GemmArgs& a, int* splits_out, hipStream_t stream) {
-    if (a.N % 64 || a.K % 64 || a.Tpad % (32 * TT) || a.cus < 8 || a.cus % 8) return hipErrorInvalidValue;
+    if (a.N % 64 || a.K % 64 || a.Tpad != 32 * TT * NB || a.cus < 8 || a.cus % 8) return hipErrorInvalidValue;
     if constexpr (EPI != EPI_PARTIAL)
-        if (a.N / 64 * (a.Tpad / (32 * TT)) >= 2 * a.cus) return launch_stream<TT, EPI, W4, 4>(a, splits_out, stream);
-    return launch_stream<TT, EPI, W4, 8>(a, splits_out, stream);
+        if (a.N / 64 * NB >= 2 * a.cus) return launch_stream<TT, NB, EPI, W4, 4>(a, splits_out, stream);
+    return launch_stream<TT, NB, EPI, W4, 8>(a, splits_out, stream);
 }
 
 constexpr int MIN_UNITS = 8;  // smallest K range worth a stream-K group
@@ -968,7 +968,7 @@ hipError_t dispatch(const GemmArgs& a, int* splits_out, hipStream_t stream) {
     switch (a.Tpad) {
         case 128:
             if constexpr (!RING64)
-                return dispatch_stream<EPI == EPI_PARTIAL ? 4 : 2, EPI, W4>(a, splits_out, stream);
+                return dispatch_stream<EPI == EPI_PARTIAL ? 4 : 2, EPI == EPI_PARTIAL ? 1 : 2, EPI, W4>(a, splits_out, stream);
             else
                 return wide ? launch<8, 1, 2, 4, A8, 3, EPI, W4, F8>(a, splits_out, stream)
                             : launch<4, 2, 2, 2, A8, 3, EPI, W4, F8>(a, splits_out, stream);
@@ -991,14 +991,14 @@ hipError_t dispatch(const GemmArgs& a, int* splits_out, hipStream_t stream) {
                 return wide ? launch<8, 1, 2, 2, A8, (A8 ? 4 : 3), EPI, W4, F8>(a, splits_out, stream)
                             : launch<4, 2, 2, 1, A8, 4, EPI, W4, F8>(a, splits_out, stream);
             } else {
-                return dispatch_stream<2, EPI, W4>(a, splits_out, stream);
+                return dispatch_stream<2, 1, EPI, W4>(a, splits_out, stream);
             }
         case 32:
             if constexpr (RING32)
                 return wide ? launch<8, 1, 2, 1, A8, 4, EPI, W4, F8>(a, splits_out, stream)
                             : launch<4, 1, 2, 1, A8, 4, EPI, W4, F8>(a, splits_out, stream);
             else
-                return dispatch_stream<1, EPI, W4>(a, splits_out, stream);
+                return dispatch_stream<1, 1, EPI, W4>(a, splits_out, stream);
         default:
             return hipErrorInvalidValue;
     }
