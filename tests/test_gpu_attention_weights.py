@@ -1,4 +1,4 @@
-"""The softmax weights of the chunked attention at the small end of float32, where the two exponentials that
+"""The softmax weights of the chunked and the prefill attention at the small end of float32, where the two exponentials that
 form them must not lose values: positions 88 below the row's maximum weigh e^-88 = 6.05e-39, below 2^-126, and with
 values of 3e35 they are all of the row's output (the other positions' values are zero)."""
 
@@ -15,7 +15,7 @@ from qwen38_amd.steps import Engine, StepGraph
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("form", ["decode"])
+@pytest.mark.parametrize("form", ["decode", "prefill"])
 def test_weights_below_the_smallest_normal_number(gpu, form):
     cfg, seq, start, chunk = probe_config(), 2048, 1500, 32  # above 1,024 positions decode takes the chunked kernels
     engine = Engine(cfg, 1, 1, seq, mtp=False, prefill_chunk=chunk)
