@@ -496,7 +496,7 @@ int run_mixer(q38_handle* h, int li, const StepIO& io, int rd, int wr, hipStream
             p.v_scale = vs;
             p.qs = (uint16_t*)h->ws(h->off_pqs);
             p.mx = (int*)h->ws(h->off_pmx);
-            p.part = (float*)h->ws(h->off_ppart);
+            p.part = (bf16_t*)h->ws(h->off_ppart);
             p.part_rows = (float*)h->ws(h->off_prows);
             p.part_slots = h->prefill_slots;
             p.k_wide = (bf16_t*)h->ws(h->off_pkw);
@@ -746,10 +746,10 @@ int q38_create(const q38_config* cfg, q38_handle** out) {
         h->off_ppt = take(Tc / PREFILL_GDN_CHUNK * h->Hv * 2 * PREFILL_GDN_CHUNK * PREFILL_GDN_CHUNK * 4);
         h->off_pdecay = take(Tc * h->Hv * 3 * 4);
         h->off_pqs = take((size_t)h->Hq * Tc * 256 * 2);
-        h->off_pmx = take((size_t)h->Hq * ((h->S + Tc + 2047) / 2048) * Tc * 4);
-        h->prefill_slots = prefill_slots(c.prefill_chunk, h->Hq, h->Hkv);
-        h->off_ppart = take(h->prefill_slots * 4 * 64 * 256 * 4);
-        h->off_prows = take(h->prefill_slots * 256 * 2 * 4);
+        h->off_pmx = take((size_t)h->Hq * prefill_blocks(Tc, h->S) * Tc * 4);
+        h->prefill_slots = prefill_slots(c.prefill_chunk, h->S, h->Hq, h->Hkv);
+        h->off_ppart = take(h->prefill_slots * 4 * 64 * 256 * 2);
+        h->off_prows = take(h->prefill_slots * 256 * 4);
         if (c.kv_cache_format == Q38_KV_FP8) {
             h->off_pkw = take((size_t)h->Hkv * h->S * 256 * 2);
             h->off_pvw = take((size_t)h->Hkv * h->S * 256 * 2);

@@ -137,24 +137,34 @@ struct PrefillAttnArgs {
     const bf16_t* k_scale;
     const bf16_t* v_scale;
     int* mx;                 // scratch [Hq][blocks of 2048 over S + L][L]: largest score per token and block, as ordered ints
-    float* part;             // scratch [part_slots][4][64][256]: an item's sums of weights x V
-    float* part_rows;        // scratch [part_slots][256][2]: an item's maximum and weight sum per token
+    bf16_t* part;            // scratch, part_slots of [4][64][256] bf16: sums of weights x V (prefill.hip, PrefillSlots)
+    float* part_rows;        // scratch [part_slots][256]: weight sums per token
     size_t part_slots;
     bf16_t* k_wide;          // kv8: scratch [Hkv][S][256], the row's keys widened
     bf16_t* v_wide;          // kv8: scratch [Hkv][S/32][256][32]
     const bf16_t* kw;        // set by the launcher: the keys and values the attention reads, and whether they hold every
     const bf16_t* vw;        // row (the caches) or only this one (the widened copies)
-    int kw_slot, ns_max, cus;
+    int kw_slot, ns_max, nblk, cus;  // most items per tile; blocks of 2048 over S + L
 };
 
-constexpr int PREFILL_RANGES = 8;   // most ranges of positions a prefill attention tile is split into
+constexpr int PREFILL_RANGES = 8;   // most items a prefill attention tile's positions are cut into
 constexpr int PREFILL_ITEMS = 768;  // most items in all, when the tiles alone are not more
-// Slots of the prefill attention's partial sums for chunks of up to L tokens: quads * min(PREFILL_RANGES,
-// max(1, PREFILL_ITEMS / quads)) with quads = Hkv * ceil(Hq / Hkv * ceil(L / 64) / 4), at its largest.
-inline size_t prefill_slots(int L, int Hq, int Hkv) {
-    const size_t quads = (size_t)Hkv * ((Hq / Hkv * ((L + 63) / 64) + 3) / 4);
-    const size_t split = quads * PREFILL_RANGES;
-    return quads > PREFILL_ITEMS ? quads : split < PREFILL_ITEMS ? split : (size_t)PREFILL_ITEMS;
+inline int prefill_blocks(int L, int S) { return (S + L + 2047) / 2048; }  // the reference's blocks of [cache, chunk]
+inline int prefill_ranges_max(int quads) {
+    const int n = quads < PREFILL_ITEMS ? PREFILL_ITEMS / quads : 1;
+    return n < PREFILL_RANGES ? n : PREFILL_RANGES;
+}
+// Slots (128 KiB) of the prefill attention's sums for chunks of up to L tokens in a cache of S: per quad of wave tiles one for
+// each block and, in float32, two for each cut between items. With 24 query heads over 4 and 2,048 tokens 12 KiB per
+// cache position, a fifth of what the 27B model's 16 attention layers keep for a position of one row, and 0.3 GB.
+inline size_t prefill_slots(int L, int S, int Hq, int Hkv) {
+    size_t most = 0;
+    for (int l = 64; l < L + 64; l += 64) {
+        const size_t quads = (size_t)Hkv * ((Hq / Hkv * (l / 64) + 3) / 4);
+        const size_t slots = quads * (prefill_blocks(l < L ? l : L, S) + 4 * (prefill_ranges_max((int)quads) - 1));
+        most = slots > most ? slots : most;
+    }
+    return most;
 }
 
 #define ATTN_KMAX 8   // verify tokens

@@ -502,8 +502,8 @@ __global__ __launch_bounds__(256) void attn_prefill_prep_kernel(const PrefillAtt
             out[e] = d < 64 ? rbf(rbf(hn[e] * cs[e]) + rbf((d < 32 ? -part : part) * sn[e])) : hn[e];
         }
         if (r < Hq) {
-            for (int b = lane; b < (S + a.L + 2047) >> 11; b += 64)  // the row's block maxima start below every score
-                a.mx[((size_t)r * ((S + a.L + 2047) >> 11) + b) * a.L + t] = order_bits(-INFINITY);
+            for (int b = lane; b < a.nblk; b += 64)  // the row's block maxima start below every score
+                a.mx[((size_t)r * a.nblk + b) * a.L + t] = order_bits(-INFINITY);
             *(uint2*)(a.qs + ((size_t)r * a.L + t) * QP + d0) =
                 make_uint2(pk_bf16(out[0] * 0.0625f, out[1] * 0.0625f), pk_bf16(out[2] * 0.0625f, out[3] * 0.0625f));
         } else if (p < S) {
@@ -530,13 +530,14 @@ __global__ __launch_bounds__(256) void attn_prefill_prep_kernel(const PrefillAtt
 // holds the position, so m has to be known before a block's first weight: attn_prefill_max makes one pass over the
 // scores for the blocks' maxima (two waves per SIMD), attn_prefill a second one for weights x V. Since every block's
 // maximum is then known, a tile's positions need not be taken in order by one workgroup: the work is dealt out as items
-// (tile of four waves, range of sub-blocks), as many ranges per tile as fill the CUs evenly (prefill_plan), and
-// attn_prefill_finish adds the ranges' float32 sums in order.
+// (tile of four waves, range of sub-blocks), as many ranges per tile as fill the CUs evenly (prefill_ranges), and
+// attn_prefill_finish puts the blocks together in order.
 //
-// Bounds: the matrix cores. 2,048 tokens after 14,336 positions of the 27B layer (24 x 256 dims): 3 x 387 GFLOP in 302 +
-// 892 + 48 us (0.93 PFLOP/s; two passes over the scores), before with 32 tokens a wave, 128 a workgroup and every tile's
-// positions in one workgroup 3,669 us. 416 tokens after 1,111 over an FP8 cache: 95 us (widening, maxima, weights x V
-// and sums), before 267.
+// Bounds: the matrix cores, and in attn_prefill the weights' exponentials beside them. 2,048 tokens after 14,336 positions of
+// the 27B layer (24 x 256 dims): 3 x 387 GFLOP in 310 + 1,120 + 110 us (0.75 PFLOP/s; two passes over the scores), before
+// with 32 tokens a wave, 128 a workgroup and every tile's positions in one workgroup 3,669 us. Items that are whole blocks
+// would save two thirds of the last kernel's reads, but leave the CUs idle: nine blocks over four items or less, 478 +
+// 1,384 + 51 us.
 namespace {
 
 constexpr int PF_ROWS = 64;                  // tokens per wave
@@ -555,17 +556,28 @@ __device__ __forceinline__ float exp_neg(float x) {
 }
 
 // Sub-blocks (of 32 aligned cache positions) a tile sees: the cached positions [0, start) in order, then its own
-// chunk's tokens 0 .. top, cut where the reference's blocks of [cache, chunk] end.
+// chunk's tokens 0 .. top, cut where the reference's blocks of [cache, chunk] end. Its blocks are numbered over those that
+// hold a position the tile may see: the cached ones, then the own tokens', the first of which the last cached one may
+// hold as well.
 struct PrefillSpan {
     int S, start, n_c, first;  // first: own tokens before the first cut
+    int cached, shared;        // blocks with cached positions; 1 if the last of them holds own tokens too
     __device__ __forceinline__ PrefillSpan(int S_, int start_)
-        : S(S_), start(start_), n_c((start_ + 31) >> 5), first(2048 - (S_ & 2047)) {}
+        : S(S_), start(start_), n_c((start_ + 31) >> 5), first(2048 - (S_ & 2047)), cached((start_ + 2047) >> 11),
+          shared(start_ > 0 && (start_ - 1) >> 11 == S_ >> 11) {}
     __device__ __forceinline__ int own(int lo, int end) const {  // sub-blocks of own tokens [lo, end)
         return end > lo ? ((start + end + 31) >> 5) - ((start + lo) >> 5) : 0;
     }
     __device__ __forceinline__ int count(int top) const {
         int n = n_c;
         for (int lo = 0, end = first; lo <= top; lo = end, end += 2048) n += own(lo, min(end, top + 1));
+        return n;
+    }
+    __device__ __forceinline__ int block_id(int j) const { return j < cached ? j : (S >> 11) + j - cached + shared; }
+    __device__ __forceinline__ int edge(int top, int j) const {  // the first sub-block of block j
+        if (j < cached) return 64 * j;
+        int n = n_c;
+        for (int i = cached - shared, lo = 0, end = first; i < j && lo <= top; ++i, lo = end, end += 2048) n += own(lo, min(end, top + 1));
         return n;
     }
 };
@@ -588,23 +600,34 @@ __device__ __forceinline__ PrefillSub prefill_sub(const PrefillSpan& sp, int top
     return {(((sp.start + lo) >> 5) + u) * 32, sp.start + lo, sp.start + min(end, top + 1), 1, (sp.S + lo) >> 11};
 }
 
-// The item of this workgroup: tile (KV head, four wave tiles) and its range [u0, u1) of sub-blocks. Ranges per tile: the
-// count up to ns_max that ends the last tile first when every CU takes items of 1 / count of the longest tile, each with
-// a fixed cost of about six sub-blocks (queries, first loads, output). Workgroups start in id order and go to the XCDs in turn:
-// ranges outermost, so that an XCD's workgroups stream the same part of one KV head (8 / Hkv XCDs per head) through its
-// L2; the tiles with the latest tokens, the longest, first.
-struct PrefillItem {
-    int kvh, quad, top, u0, u1, ns, z;
-};
-
-__device__ __forceinline__ bool prefill_item(const PrefillAttnArgs& a, const PrefillSpan& sp, int id, PrefillItem& it) {
-    const int G = a.Hq / a.Hkv, ntt = (a.L + PF_ROWS - 1) / PF_ROWS, nq = (G * ntt + 3) / 4;
-    const int longest = sp.count(a.L - 1), tiles = nq * a.Hkv;
+// Items (ranges of sub-blocks) per tile: the count up to ns_max that ends the last tile first when every CU takes items of
+// 1 / count of the longest tile, each with a fixed cost of about six sub-blocks (queries, first loads, output).
+__device__ __forceinline__ int prefill_ranges(const PrefillAttnArgs& a, const PrefillSpan& sp) {
+    const int tiles = (a.Hq / a.Hkv * ((a.L + PF_ROWS - 1) / PF_ROWS) + 3) / 4 * a.Hkv, longest = sp.count(a.L - 1);
     int ns = 1, best = 0x7fffffff;
     for (int c = 1; c <= a.ns_max && (c == 1 || longest >= 4 * c); ++c) {
         const int cost = ((tiles * c + a.cus - 1) / a.cus) * ((longest + c - 1) / c + 6);
         if (cost < best) best = cost, ns = c;
     }
+    return ns;
+}
+
+__device__ __forceinline__ int prefill_cut(int n, int z, int ns) { return z * n / ns; }  // where item z of n sub-blocks starts
+
+__device__ __forceinline__ int prefill_top(const PrefillAttnArgs& a, int quad) {  // the last token of the quad's tiles
+    const int G = a.Hq / a.Hkv, ntt = (a.L + PF_ROWS - 1) / PF_ROWS;
+    return min((min(quad * 4 + 3, G * ntt - 1) / G) * PF_ROWS + PF_ROWS - 1, a.L - 1);
+}
+
+// The item of this workgroup: tile (KV head, four wave tiles), its range z of sub-blocks, [u0, u1). Workgroups start in id
+// order and go to the XCDs in turn: ranges outermost, so that an XCD's workgroups stream the same part of one KV head
+// (8 / Hkv XCDs per head) through its L2; the tiles with the latest tokens, the longest, first.
+struct PrefillItem {
+    int kvh, quad, top, u0, u1, z;
+};
+
+__device__ __forceinline__ bool prefill_item(const PrefillAttnArgs& a, const PrefillSpan& sp, int id, PrefillItem& it) {
+    const int nq = (a.Hq / a.Hkv * ((a.L + PF_ROWS - 1) / PF_ROWS) + 3) / 4, ns = prefill_ranges(a, sp);
     int j;
     if (a.Hkv <= 8 && 8 % a.Hkv == 0) {
         const int per = 8 / a.Hkv, x = id & 7;
@@ -615,22 +638,33 @@ __device__ __forceinline__ bool prefill_item(const PrefillAttnArgs& a, const Pre
         j = id / a.Hkv;
     }
     if (j >= nq * ns) return false;
-    it.ns = ns;
     it.z = j / nq;
     it.quad = nq - 1 - j % nq;
-    const int last = min(it.quad * 4 + 3, G * ntt - 1);  // the quad's last tile with tokens
-    it.top = min((last / G) * PF_ROWS + PF_ROWS - 1, a.L - 1);
+    it.top = prefill_top(a, it.quad);
     const int n = sp.count(it.top);
-    it.u0 = (int)((long)it.z * n / ns);
-    it.u1 = (int)((long)(it.z + 1) * n / ns);
+    it.u0 = prefill_cut(n, it.z, ns);
+    it.u1 = prefill_cut(n, it.z + 1, ns);
     return true;
 }
 
-// Partial slots: (KV head, quad, range), of 4 waves x 64 tokens x 256 dims floats, and 2 floats per token.
-__device__ __forceinline__ size_t prefill_slot(const PrefillAttnArgs& a, int kvh, int quad, int z) {
-    const int nq = (a.Hq / a.Hkv * ((a.L + PF_ROWS - 1) / PF_ROWS) + 3) / 4;
-    return (size_t)(kvh * nq + quad) * a.ns_max + z;
-}
+// Where a quad's sums go. A block that one item has all of: slot j (the block) of nblk, 4 waves x 64 tokens x 256 dims in
+// bf16, rounded as the reference rounds each block's weights x V. A block that cuts divide: the parts' float32 sums, in two
+// slots per cut between items: 2 (z - 1) + 1 for what item z begins with, 2 z for what it ends with (a part that begins
+// and ends an item counts as its beginning). Beside each slot a float per token, its weight sum.
+struct PrefillSlots {
+    bf16_t* blocks;
+    float *parts, *rows;  // [nblk + 2 (ns_max - 1)][4 waves][64 tokens]
+    int nblk;
+    __device__ __forceinline__ PrefillSlots(const PrefillAttnArgs& a, int kvh, int quad) : nblk(a.nblk) {
+        const int nq = (a.Hq / a.Hkv * ((a.L + PF_ROWS - 1) / PF_ROWS) + 3) / 4, np = 2 * (a.ns_max - 1);
+        const size_t q = (size_t)(kvh * nq + quad), one = 4 * PF_ROWS * 256;
+        blocks = a.part + q * (a.nblk + 2 * np) * one;
+        parts = (float*)(blocks + a.nblk * one);
+        rows = a.part_rows + q * (a.nblk + np) * (4 * PF_ROWS);
+    }
+    // The part of a block that item z holds: `later` if a cut lies before it in the block.
+    __device__ __forceinline__ static int part(int z, bool later) { return later ? 2 * z - 1 : 2 * z; }
+};
 
 __device__ __forceinline__ float order_float(int i) { return __int_as_float(i >= 0 ? i : i ^ 0x7fffffff); }
 
@@ -755,14 +789,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if (i < n) cp.keys(prefill_sub(sp, it.top, it.u0 + i).p0, lds0 + i * PF_SUB);
     const uint32_t kl = (lane & 31) * 512 + (lane >> 5) * 256 + ((lane & 15) << 4);
     float mx[2] = {-INFINITY, -INFINITY};
-    const int nblk = (a.S + a.L + 2047) >> 11;
     auto flush = [&](int block) {
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt) {
             // The largest bf16 score is the largest score in bf16.
             const float m = rbf(fmaxf(mx[rt], __shfl_xor(mx[rt], 32)));
             const int t = tl.t0 + rt * 32 + (lane & 31);
-            if (lane < 32 && tl.live && t < a.L && m > -INFINITY) atomicMax(a.mx + ((size_t)tl.hq * nblk + block) * a.L + t, order_bits(m));
+            if (lane < 32 && tl.live && t < a.L && m > -INFINITY) atomicMax(a.mx + ((size_t)tl.hq * a.nblk + block) * a.L + t, order_bits(m));
             mx[rt] = -INFINITY;
         }
     };
@@ -787,8 +820,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 // Weights x V of one item: per sub-block the scores again, the weights e^(s - m) with m the running maximum through the
-// sub-block's block, their float32 sums, and the bf16 weights times V; at a block's end the sums so far are rescaled
-// to the next block's maximum. V as A and the weights as B, so that a lane holds four consecutive dims of one token
+// sub-block's block, their float32 sums, and the bf16 weights times V; at a block's end the block's sums go to its
+// slot, a whole block's rounded to bf16. V as A and the weights as B, so that a lane holds four consecutive dims of one token
 // (the order the activation tiles and the float4 partials want) and its row factors are its own. Sub-block i's
 // weights x V run beside sub-block i + 1's scores, whose weights are formed beside them (the loop body has no branch
 // but the edges), with the copies two sub-blocks ahead.
@@ -801,6 +834,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     PrefillItem it;
     if (!prefill_item(a, sp, blockIdx.x, it)) return;
     const int n = it.u1 - it.u0;
+    if (n <= 0) return;
     const PrefillTile tl = prefill_tile(a, it.kvh, it.quad * 4 + wv);
     const uint32_t lds0 = (uint32_t)(uintptr_t)LDS_PTR(&ring[0][0][0]);
     SubCopy cp;
@@ -818,25 +852,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const int fd = ((lane >> 1) & 3) ^ ((lane >> 3) & 1);
     const uint32_t vl = PF_SUB + (lane & 31) * 64 + (((lane >> 5) ^ fd) << 4);
 
-    const int nblk = (a.S + a.L + 2047) >> 11;
     float nb[2] = {2.0f * -1e4f, 2.0f * -1e4f}, total[2] = {0.0f, 0.0f};
     int known = -1;  // blocks whose maxima nb holds
     auto raise = [&](int block) {
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt) {
-            const int* mp = a.mx + (size_t)tl.hq * nblk * a.L + min(tl.t0 + rt * 32, a.L - 32) + (lane & 31);
+            const int* mp = a.mx + (size_t)tl.hq * a.nblk * a.L + min(tl.t0 + rt * 32, a.L - 32) + (lane & 31);
             if (tl.live)
                 for (int b = known + 1; b <= block; ++b) nb[rt] = fmaxf(nb[rt], order_float(mp[(size_t)b * a.L]));
         }
         known = block;
     };
     v16f o[2][8];  // o[rt][db][e]: token 32 rt + l % 32, dim 32 db + 8 (e / 4) + 4 (l / 32) + e % 4
-#pragma unroll
-    for (int rt = 0; rt < 2; ++rt)
-#pragma unroll
-        for (int db = 0; db < 8; ++db)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) o[rt][db][e] = 0.0f;
     v16f s[2];
     // Two of the sub-block's weights (x: token tile x / 8, MFMA step x / 4 % 2, word x % 4) into w.
     typedef uint32_t u4_ __attribute__((ext_vector_type(4)));
@@ -889,24 +916,48 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         const PrefillSub sb = prefill_sub(sp, it.top, it.u0 + i);
         if (!prefill_whole(sb, tl, start)) prefill_mask(sb, tl, start, lane, s);
     };
-    // One block of the reference at a time: between them the sums are rescaled, so the inner loop only accumulates.
-    for (int i = 0; i < n;) {
-        const int block = prefill_sub(sp, it.top, it.u0 + i).block;
-        int end = i + 1;  // this block's sub-blocks end here
-        if (it.u0 + i < sp.n_c) end = min(n, min(sp.n_c, (it.u0 + i | 63) + 1) - it.u0);
-        while (end < n && prefill_sub(sp, it.top, it.u0 + end).block == block) ++end;
-        const float b0 = nb[0], b1 = nb[1];
-        raise(block);
-        if (i > 0) {
-            const float f[2] = {exp_neg(b0 - nb[0]), exp_neg(b1 - nb[1])};
+    // The sums of block j, or of a part of it, [wave][rt][db][e / 4][lane] of 4 dims, and per token its weight sum.
+    const PrefillSlots slots(a, it.kvh, it.quad);
+    auto store = [&](int j, bool whole, bool later) __attribute__((always_inline)) {
+        const int part = PrefillSlots::part(it.z, later);
+        const size_t at = (size_t)(whole ? j : part) * (4 * PF_ROWS * 256) + (size_t)wv * (PF_ROWS * 256) + lane * 4;
+        if (whole) {
 #pragma unroll
-            for (int rt = 0; rt < 2; ++rt) {
-                total[rt] *= f[rt];
+            for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
                 for (int db = 0; db < 8; ++db)
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) o[rt][db][e] *= f[rt];
-            }
+                    for (int q = 0; q < 4; ++q)
+                        *(uint2*)(slots.blocks + at + ((rt * 8 + db) * 4 + q) * 256) =
+                            make_uint2(pk_bf16(o[rt][db][4 * q], o[rt][db][4 * q + 1]), pk_bf16(o[rt][db][4 * q + 2], o[rt][db][4 * q + 3]));
+        } else {
+#pragma unroll
+            for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+                for (int db = 0; db < 8; ++db)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        *(v4f*)(slots.parts + at + ((rt * 8 + db) * 4 + q) * 256) =
+                            (v4f){o[rt][db][4 * q], o[rt][db][4 * q + 1], o[rt][db][4 * q + 2], o[rt][db][4 * q + 3]};
+        }
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) {
+            const float sum = total[rt] + __shfl_xor(total[rt], 32);
+            if (lane < 32) slots.rows[(whole ? j : slots.nblk + part) * (4 * PF_ROWS) + wv * PF_ROWS + rt * 32 + lane] = sum;
+        }
+    };
+    int j = 0;  // the block of the item's first sub-block
+    while (sp.edge(it.top, j + 1) <= it.u0) ++j;
+    for (int i = 0; i < n; ++j) {  // one block at a time
+        const int e0 = sp.edge(it.top, j) - it.u0, e1 = sp.edge(it.top, j + 1) - it.u0, first = i, end = min(n, e1);
+        raise(sp.block_id(j));
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) {
+            total[rt] = 0.0f;
+#pragma unroll
+            for (int db = 0; db < 8; ++db)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) o[rt][db][e] = 0.0f;
         }
         scores(i);
 #pragma unroll
@@ -916,28 +967,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             values(i, std::true_type{});
         }
         values(i++, std::false_type{});
-    }
-    if (!tl.live) return;
-    // The range's sums, [wave][rt][db][e / 4][lane] float4, and per token its maximum and weight sum.
-    const size_t sl = prefill_slot(a, it.kvh, it.quad, it.z);
-    float* po = a.part + sl * (4 * PF_ROWS * 256) + (size_t)wv * (PF_ROWS * 256) + lane * 4;
-#pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-#pragma unroll
-        for (int db = 0; db < 8; ++db)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                *(v4f*)(po + ((rt * 8 + db) * 4 + q) * 256) =
-                    (v4f){o[rt][db][4 * q], o[rt][db][4 * q + 1], o[rt][db][4 * q + 2], o[rt][db][4 * q + 3]};
-        const float sum = total[rt] + __shfl_xor(total[rt], 32);
-        if (lane < 32) *(float2*)(a.part_rows + (sl * 4 * PF_ROWS + wv * PF_ROWS + rt * 32 + lane) * 2) = make_float2(nb[rt], sum);
+        if (tl.live) store(j, first == e0 && end == e1, first > e0);
     }
 }
 
-// The ranges of one wave tile added in order, out / total in bf16, times bf16 sigmoid(gate), e5m2 tiles for o_proj. Grid
-// (wave tiles of 64 tokens x 4): wave w of block q takes 32 tokens and 64 dims, a lane 4 dims of one token at a time. The
-// reference rounds each block's weights x V to bf16; with all of a token's positions in one block that rounding is the
-// sum's, and kept, and over several blocks the float32 sums are used as they are.
+// One wave tile's blocks put together as the reference does: from block to block the sums so far are rescaled to the running
+// maximum and the block's weights x V, rounded to bf16, added in float32; then out / total in bf16, times bf16
+// sigmoid(gate), e5m2 tiles for o_proj. Grid (wave tiles of 64 tokens x 4): wave w of block q takes 32 tokens and 64 dims, a
+// lane 4 dims of one token at a time.
 __global__ __launch_bounds__(256) void attn_prefill_finish_kernel(const PrefillAttnArgs a) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int slot = *a.slot, start = *a.start;
@@ -945,30 +982,58 @@ __global__ __launch_bounds__(256) void attn_prefill_finish_kernel(const PrefillA
     const PrefillSpan sp(a.S, start);
     const int G = a.Hq / a.Hkv, ntt = (a.L + PF_ROWS - 1) / PF_ROWS;
     const int kvh = blockIdx.y, tile = blockIdx.x >> 2, quad = tile >> 2, w = tile & 3;
-    PrefillItem it;
-    if (tile >= G * ntt || !prefill_item(a, sp, 0, it)) return;
+    if (tile >= G * ntt) return;
     const PrefillTile tl = prefill_tile(a, kvh, tile);
     const int rt = wv & 1, db0 = ((blockIdx.x & 3) * 2 + (wv >> 1)), t = tl.t0 + rt * 32 + (lane & 31);
     if (tl.t0 + rt * 32 >= a.L) return;
-    const size_t sl = prefill_slot(a, kvh, quad, 0);
-    const float* rows = a.part_rows + (sl * 4 * PF_ROWS + w * PF_ROWS + rt * 32 + (lane & 31)) * 2;
-    const float M = rows[(size_t)(it.ns - 1) * 4 * PF_ROWS * 2];  // the last range's maximum is the largest
-    const bool one = (start == 0 || start <= 2048) && (a.S + t) >> 11 == (start > 0 ? 0 : a.S >> 11);
-    float total = 0.0f;
+    const int top = prefill_top(a, quad);
+    const int n = sp.count(top), ns = prefill_ranges(a, sp);
+    const PrefillSlots slots(a, kvh, quad);
+    const float* rows = slots.rows + w * PF_ROWS + rt * 32 + (lane & 31);
+    const size_t at = (size_t)w * (PF_ROWS * 256) + (rt * 8 + db0) * 1024 + lane * 4;
+    const int* mp = a.mx + (size_t)tl.hq * a.nblk * a.L + t;
+    float best = 2.0f * -1e4f, total = 0.0f;
     v4f o[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) o[q] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
-    for (int z = 0; z < it.ns; ++z) {
-        const float2 r = *(const float2*)(rows + (size_t)z * 4 * PF_ROWS * 2);
-        const float f = exp_neg(r.x - M);
-        total += r.y * f;
-        const float* po = a.part + (sl + z) * (4 * PF_ROWS * 256) + (size_t)w * (PF_ROWS * 256) + (rt * 8 + db0) * 1024 + lane * 4;
+    int z = 0;  // the item that holds the block's first sub-block
+    for (int j = 0, e0 = 0; e0 < n; ++j) {
+        const int e1 = sp.edge(top, j + 1);
+        const float m = fmaxf(best, order_float(mp[(size_t)sp.block_id(j) * a.L])), f = exp_neg(best - m);
+        best = m;
+        float sum = 0.0f;
+        v4f pv[4];
+        while (prefill_cut(n, z + 1, ns) <= e0) ++z;
+        if (prefill_cut(n, z + 1, ns) >= e1) {
+            sum = rows[j * (4 * PF_ROWS)];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const v4f v = *(const v4f*)(po + q * 256);
+            for (int q = 0; q < 4; ++q) {
+                const uint2 v = *(const uint2*)(slots.blocks + (size_t)j * (4 * PF_ROWS * 256) + at + q * 256);
+                pv[q] = (v4f){lo_bf(v.x), hi_bf(v.x), lo_bf(v.y), hi_bf(v.y)};
+            }
+        } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[q][e] += v[e] * f;
+            for (int q = 0; q < 4; ++q) pv[q] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+            for (int y = z, u0 = prefill_cut(n, z, ns); u0 < e1; ++y) {
+                const int u1 = prefill_cut(n, y + 1, ns), part = PrefillSlots::part(y, u0 > e0);
+                if (u1 > u0) {  // else the item is empty
+                    sum += rows[(slots.nblk + part) * (4 * PF_ROWS)];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) pv[q] += *(const v4f*)(slots.parts + (size_t)part * (4 * PF_ROWS * 256) + at + q * 256);
+                }
+                u0 = u1;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) pv[q][e] = rbf(pv[q][e]);
         }
+        total = total * f + sum;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[q][e] = o[q][e] * f + pv[q][e];
+        e0 = e1;
     }
     const int act_k = a.Hq * 256;
 #pragma unroll
@@ -979,7 +1044,7 @@ __global__ __launch_bounds__(256) void attn_prefill_finish_kernel(const PrefillA
         float r[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float v = rbf((one ? rbf(o[q][e]) : o[q][e]) / total);
+            const float v = rbf(o[q][e] / total);
             r[e] = rbf(v * rbf(sigmoidf_(gt[e])));
         }
         *(uint32_t*)(a.act + act_offset(t, tl.hq * 256 + d, act_k)) = pk_e5m2(r[0], r[1], r[2], r[3]);
@@ -1005,6 +1070,7 @@ __global__ __launch_bounds__(256) void attn_prefill_widen_kernel(const PrefillAt
 
 hipError_t q38_attn_prefill(const PrefillAttnArgs& a0, hipStream_t stream) {
     PrefillAttnArgs a = a0;
+    a.nblk = prefill_blocks(a.L, a.S);
     if (a.L < 1 || a.L % 32 || a.Hq % a.Hkv || a.S % 32) return hipErrorInvalidValue;
     if (a.kv8 && (!a.k_scale || !a.v_scale)) return hipErrorInvalidValue;
     if (a.kv8)
@@ -1013,9 +1079,9 @@ hipError_t q38_attn_prefill(const PrefillAttnArgs& a0, hipStream_t stream) {
         hipLaunchKernelGGL(attn_prefill_prep_kernel<false>, dim3(a.L), dim3(256), 0, stream, a);
     if (a.keys_only) return hipGetLastError();
     const int tiles = (a.Hq / a.Hkv) * ((a.L + PF_ROWS - 1) / PF_ROWS), quads = (tiles + 3) / 4 * a.Hkv;
-    a.ns_max = std::min(PREFILL_RANGES, std::max(1, PREFILL_ITEMS / quads));
+    a.ns_max = prefill_ranges_max(quads);
     a.cus = q38_device_cus();
-    if ((size_t)quads * a.ns_max > a.part_slots) return hipErrorInvalidValue;
+    if ((size_t)quads * (a.nblk + 4 * (a.ns_max - 1)) > a.part_slots) return hipErrorInvalidValue;
     a.kw = a.k_cache;
     a.vw = a.v_cache;
     a.kw_slot = 1;
