@@ -39,10 +39,11 @@ __device__ __forceinline__ float conv_window(const PrefillGdnArgs& a, const bf16
 
 __device__ __forceinline__ v4f mfma16(float x, float y, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0); }
 
-// e^x of a 64-bit x, in float32 without x's own rounding (|x| ulps of the result).
-__device__ __forceinline__ float exp_of(double x) {
-    const float hi = (float)x, e = expf(hi);
-    return e + e * (float)(x - hi);
+// e^x of a 64-bit x, to expf's error without x's own rounding (|x| ulps of the result).
+__device__ __forceinline__ double exp_of(double x) {
+    const float hi = (float)x;
+    const double e = expf(hi);
+    return e + e * (x - hi);
 }
 
 // This wave's LDS accesses are done; then meet the other waves (loads from global memory stay in flight).
@@ -51,13 +52,13 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 }  // namespace
 
 // Grid (32 tokens, key head): conv, SiLU, l2 norms and gates of the tokens, then what a chunk of the delta rule needs that
-// does not depend on the state. With c_t the log decays summed from the chunk's start, k . k and q . k on the float32 MFMA, and per
+// does not depend on the state. With c_t the log decays summed from the chunk's start, k . k and q . k on the float64 MFMA, and per
 // value head M_ts = beta_t e^(c_t - c_s) k_t . k_s (s < t), T = (I + M)^-1 by forward substitution (a column per lane),
 // P_ts = e^(c_t - c_s) q_t . k_s (s <= t).
 // Bounds: the conv's and SiLU's arithmetic (about 40 instructions per input at a bf16 rounding after each operation; the
 // memory traffic, 145 MB for 2,048 tokens of the 27B layer, is half its time). Wave w takes tokens 8 w .. 8 w + 7 of one
 // head after another, a lane two channels, each input loaded once for the four taps, the next head's meanwhile: 60 us
-// with the matrices, where one token and channel per thread took 152 us for the conv and norms alone.
+// with the matrices (67 since these are 64-bit sums), where one token and channel per thread took 152 us for the conv and norms alone.
 __global__ __launch_bounds__(256) void gdn_prefill_prep_kernel(const PrefillGdnArgs a) {
     constexpr int D = 128, GMAX = 8, KP = D + 4, MP = GC + 4;
     __shared__ __attribute__((aligned(16))) float sk[GC][KP], sq[GC][KP], sm[4][GC][MP];
@@ -142,9 +143,11 @@ __global__ __launch_bounds__(256) void gdn_prefill_prep_kernel(const PrefillGdnA
     __syncthreads();
 
     // k . k and q . k, a 16 x 16 quarter per wave (rows t, columns s; the quarter above the diagonal stays zero): four
-    // MFMA steps per 16-byte read, the same order of inputs in both operands.
+    // MFMA steps per 16-byte read, the same order of inputs in both operands. In 64 bits: as float32 chains of 128 their
+    // rounding was most of the delta rule's error.
     const int wr = wave >> 1, wc = wave & 1, lr = lane & 15, lq = lane >> 4;
-    v4f kk = {0.0f, 0.0f, 0.0f, 0.0f}, qk = kk;
+    typedef double v4d __attribute__((ext_vector_type(4)));
+    v4d kk = {0.0, 0.0, 0.0, 0.0}, qk = kk;  // element i: row 16 wr + 4 i + lq, column 16 wc + lr
     if (wr >= wc)
 #pragma unroll
         for (int g = 0; g < 8; ++g) {
@@ -152,8 +155,8 @@ __global__ __launch_bounds__(256) void gdn_prefill_prep_kernel(const PrefillGdnA
             const v4f ks = *(const v4f*)&sk[16 * wc + lr][16 * g + 4 * lq];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                kk = mfma16(kt[e], ks[e], kk);
-                qk = mfma16(qt[e], ks[e], qk);
+                kk = __builtin_amdgcn_mfma_f64_16x16x4f64(kt[e], ks[e], kk, 0, 0, 0);
+                qk = __builtin_amdgcn_mfma_f64_16x16x4f64(qt[e], ks[e], qk, 0, 0, 0);
             }
         }
     for (int r0 = 0; r0 < rep; r0 += 4) {  // value heads, four at a time
@@ -183,8 +186,8 @@ __global__ __launch_bounds__(256) void gdn_prefill_prep_kernel(const PrefillGdnA
             const double last = __shfl(c, 31, 32) - c;
             float* f = a.decay + (((size_t)ch * Hv + h) * 3) * GC + (tid & 31);
             f[0] = beta;
-            f[GC] = exp_of(c);
-            f[2 * GC] = exp_of(last);
+            f[GC] = (float)exp_of(c);
+            f[2 * GC] = (float)exp_of(last);
         }
         __syncthreads();
         for (int r = 0; r < nh; ++r) {
@@ -192,10 +195,10 @@ __global__ __launch_bounds__(256) void gdn_prefill_prep_kernel(const PrefillGdnA
             const int s = 16 * wc + lr;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int t = 16 * wr + 4 * lq + i;
-                const float e = t >= s ? exp_of(sc[r][t] - sc[r][s]) : 0.0f;
-                sm[r][t][s] = sb[r][t] * e * kk[i];
-                P[t * GC + s] = e * qk[i];
+                const int t = 16 * wr + 4 * i + lq;
+                const double e = t >= s ? exp_of(sc[r][t] - sc[r][s]) : 0.0;
+                sm[r][t][s] = (float)(sb[r][t] * e * kk[i]);
+                P[t * GC + s] = (float)(e * qk[i]);
             }
         }
         __syncthreads();
@@ -229,9 +232,10 @@ __global__ __launch_bounds__(256) void gdn_prefill_prep_kernel(const PrefillGdnA
 // model.py:88-124); 32 keep T and P small, and the state's products, which are most of the work, do not depend on it.
 // Bounds: the float32 matrix rate of the CUs that 4 Hv workgroups fill: per wave and chunk 32 + 16 MFMAs of 64 cycles and
 // 16 of 32, with three LDS round trips between them. k, q, T, P, v and the gates of the next chunk load meanwhile.
-// 2,048 tokens of the 27B layer (64 chunks): 218 us, 49 TFLOP/s; token by token (one state column in 8 lanes, DPP
-// sums) 781 us. Against 64 bits from the same k, q, v, beta and g, o before its rounding to bf16 is off by
-// 1.8e-7 (1.0e-7 token by token) and after it by 1.658e-3, the state by 1.66e-3, as before.
+// 2,048 tokens of the 27B layer (64 chunks): 228 us, 47 TFLOP/s; token by token (one state column in 8 lanes, DPP
+// sums) 781 us. Against 64 bits from the same k, q, v, beta and g, o before its rounding to bf16 is off by 7.6e-8 to 1.9e-7
+// (512 tokens, decays from e^-5 to e^-0.002 per token; 7.9e-8 to 4.3e-7 token by token, and with k . k and q . k as float32
+// chains 1.7e-7 to 2.3e-7, 10 us less in all), the state after its rounding by 1.64e-3 to 1.67e-3 in every form.
 __global__ __launch_bounds__(256) void gdn_prefill_scan_kernel(const PrefillGdnArgs a) {
     constexpr int D = 128, KB = GC * D * 4, RP = 36;  // bytes of a chunk's k or q, floats per row of the 32 x 32 tiles
     __shared__ __attribute__((aligned(1024))) uint8_t ring[2][2][KB];  // [stage][k, q], 16-byte chunk c of row r at c ^ (r % 16)
@@ -313,17 +317,19 @@ __global__ __launch_bounds__(256) void gdn_prefill_scan_kernel(const PrefillGdnA
         __builtin_amdgcn_sched_barrier(0);
         if (c + 1 < nch) load(c + 1);
 
-        // k . S and q . S over this wave's 32 state rows.
-        v16f ks, qs;
+        // k . S and q . S over this wave's 32 state rows; q . S, which goes straight into o, as two sums of 16.
+        v16f ks, qs, qs2;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) ks[i] = qs[i] = 0.0f;
+        for (int i = 0; i < 16; ++i) ks[i] = qs[i] = qs2[i] = 0.0f;
 #pragma unroll
         for (int g = 0; g < 4; ++g)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 ks = __builtin_amdgcn_mfma_f32_32x32x2f32(kp[g][e], S[4 * g + e], ks, 0, 0, 0);
-                qs = __builtin_amdgcn_mfma_f32_32x32x2f32(qp[g][e], S[4 * g + e], qs, 0, 0, 0);
+                v16f& q = g < 2 ? qs : qs2;
+                q = __builtin_amdgcn_mfma_f32_32x32x2f32(qp[g][e], S[4 * g + e], q, 0, 0, 0);
             }
+        qs += qs2;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             *(v4f*)red[wave][0][q][lane] = (v4f){ks[4 * q], ks[4 * q + 1], ks[4 * q + 2], ks[4 * q + 3]};
@@ -375,13 +381,15 @@ __global__ __launch_bounds__(256) void gdn_prefill_scan_kernel(const PrefillGdnA
 #pragma unroll
         for (int i = 0; i < 4; ++i) oq[i] = sO[16 * wr + 4 * lq + i][16 * wc + lr];
         __builtin_amdgcn_sched_barrier(0);
-        v4f op[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+        v4f op[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) op[j] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
             S = __builtin_amdgcn_mfma_f32_32x32x2f32(kt[j], dw[j], S, 0, 0, 0);
-            if (j < 8) op[j >> 2] = mfma16(Pc[j >> 2][j & 3], dd[j], op[j >> 2]);
+            if (j < 8) op[j >> 1] = mfma16(Pc[j >> 2][j & 3], dd[j], op[j >> 1]);
         }
-        const v4f o = oq + (op[0] + op[1]);
+        const v4f o = oq + ((op[0] + op[1]) + (op[2] + op[3]));
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             a.o[((size_t)(c * GC + 16 * wr + 4 * lq + i) * Hv + h) * D + grp * 32 + 16 * wc + lr] = f2bf(o[i]);

@@ -10,6 +10,7 @@ token (several such steps in each of three projections), 2e-2 over all tokens, 1
 
 from __future__ import annotations
 
+import ctypes
 from dataclasses import replace
 
 import pytest
@@ -65,3 +66,50 @@ def test_a_chunk_of_the_delta_rule(gpu, key_heads, value_heads, chunk, start, n_
         print(f"{key} {err:.2e}")
         assert err <= 1e-2
         assert torch.equal(value[1 - slot], before[key][1 - slot].float())
+
+
+class PrefillGdnArgs(ctypes.Structure):
+    """csrc/kernels.h: the launcher's argument block."""
+
+    _fields_ = (
+        [(n, ctypes.c_int) for n in ("L", "Hk", "Hv", "C", "rows")]
+        + [(n, ctypes.c_void_p) for n in ("slot", "start", "n_valid", "qkv", "z", "gate_part")]
+        + [("gate_groups", ctypes.c_int)]
+        + [(n, ctypes.c_void_p) for n in ("a_log", "dt_bias", "conv_w", "norm_w", "state", "conv", "qn", "kn", "v", "decay", "pt", "o", "act")]
+        + [("eps", ctypes.c_float)]
+    )
+
+
+@pytest.mark.gpu
+def test_the_chunks_matrices_are_rounded_once(gpu):
+    """P_ts = e^(c_t - c_s) q_t . k_s and T = (I + beta k . k)^-1 of every chunk against 64 bits from the kernel's own q, k and
+    beta, without decay (A_log = -inf): an entry of P is its exact sum rounded once, 2^-24 of it, where a float32 chain of
+    128 products is off by 128 x 2^-24 of its terms at worst."""
+    L, Hk, Hv, D = 96, 2, 8, 128
+    C, rep, g = 2 * Hk * D + Hv * D, Hv // Hk, torch.Generator(device="cuda").manual_seed(5)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    ints = lambda v: torch.tensor([v], dtype=torch.int32, device="cuda")  # noqa: E731
+    zeros = lambda n: torch.zeros(n, device="cuda")  # noqa: E731
+    bf = lambda t: t.to(torch.bfloat16)  # noqa: E731
+    t = {
+        "slot": ints(0), "start": ints(0), "n_valid": ints(L), "qkv": bf(rand(L, C)), "z": bf(rand(L, Hv * D)),
+        "gate_part": rand(L, 2 * Hv), "a_log": bf(torch.full((Hv,), -torch.inf, device="cuda")), "dt_bias": bf(zeros(Hv)),
+        "conv_w": bf(rand(C, 4) * 0.5), "norm_w": bf(zeros(D)), "state": bf(zeros(Hv * D * D)), "conv": bf(zeros(C * 3)),
+        "qn": zeros(L * Hk * D), "kn": zeros(L * Hk * D), "v": bf(zeros(L * Hv * D)), "decay": zeros(L * Hv * 3),
+        "pt": zeros(L * Hv * 2 * 32), "o": bf(zeros(L * Hv * D)), "act": torch.zeros(L * Hv * D, dtype=torch.uint8, device="cuda"),
+    }
+    a = PrefillGdnArgs(L=L, Hk=Hk, Hv=Hv, C=C, rows=1, gate_groups=1, eps=1e-6, **{n: v.data_ptr() for n, v in t.items()})
+    launch = gpu["_Z15q38_gdn_prefillRK14PrefillGdnArgsP12ihipStream_t"]
+    torch.cuda.synchronize()
+    assert launch(ctypes.byref(a), ctypes.c_void_p(0)) == 0
+    torch.cuda.synchronize()
+    heads = lambda n: t[n].view(L // 32, 32, Hk, D).double().permute(0, 2, 1, 3).repeat_interleave(rep, 1).contiguous()  # noqa: E731
+    q, k, beta = heads("qn"), heads("kn"), t["decay"].view(L // 32, Hv, 3, 32)[:, :, 0].double()
+    pt = t["pt"].view(L // 32, Hv, 2, 32, 32).double()
+    want = (q @ k.transpose(-1, -2).contiguous()).tril()
+    off = (pt[:, :, 1] - want).abs()
+    print(f"P off by at most {float((off / want.abs().clamp_min(1e-30)).max()):.2e}, rms {float(off.norm() / want.norm()):.2e}")
+    assert bool((off <= 2.0**-24 * want.abs() * (1 + 1e-6)).all())
+    inverse = torch.linalg.inv(torch.eye(32, device="cuda", dtype=torch.float64) + (k @ k.transpose(-1, -2).contiguous()).tril(-1) * beta.unsqueeze(-1))
+    # Forward substitution in float32: 32 products and sums per entry.
+    assert float((pt[:, :, 0] - inverse).norm() / inverse.norm()) <= 32 * 2.0**-24
