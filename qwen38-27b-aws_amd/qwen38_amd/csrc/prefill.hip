@@ -46,6 +46,8 @@ __device__ __forceinline__ double exp_of(double x) {
     return e + e * (x - hi);
 }
 
+__device__ __forceinline__ bool finite(float x) { return fabsf(x) < INFINITY; }
+
 // This wave's LDS accesses are done; then meet the other waves (loads from global memory stay in flight).
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
@@ -174,8 +176,9 @@ __global__ __launch_bounds__(256) void gdn_prefill_prep_kernel(const PrefillGdnA
                     sum[1] += p[Hv];
                 }
             const float beta = rbf(sigmoidf_(rbf(sum[0]))) * valid;
+            const float g = -expf(bf2f(a.a_log[h])) * softplusf_(rbf(sum[1]) + bf2f(a.dt_bias[h])) * valid;
             // Summed in 64 bits: the factors are e to differences of these sums, often small ones of large ones.
-            double c = -expf(bf2f(a.a_log[h])) * softplusf_(rbf(sum[1]) + bf2f(a.dt_bias[h])) * valid;
+            double c = g;
 #pragma unroll
             for (int o = 1; o < 32; o <<= 1) {
                 const double up = __shfl_up(c, o, 32);
@@ -198,7 +201,7 @@ __global__ __launch_bounds__(256) void gdn_prefill_prep_kernel(const PrefillGdnA
                 const int t = 16 * wr + 4 * i + lq;
                 const double e = t >= s ? exp_of(sc[r][t] - sc[r][s]) : 0.0;
                 sm[r][t][s] = (float)(sb[r][t] * e * kk[i]);
-                P[t * GC + s] = (float)(e * qk[i]);
+                P[t * GC + s] = t >= s ? (float)(e * qk[i]) : 0.0f;  // not 0 q . k: a token's NaN is not an earlier one's
             }
         }
         __syncthreads();
@@ -232,7 +235,9 @@ __global__ __launch_bounds__(256) void gdn_prefill_prep_kernel(const PrefillGdnA
 // model.py:88-124); 32 keep T and P small, and the state's products, which are most of the work, do not depend on it.
 // Bounds: the float32 matrix rate of the CUs that 4 Hv workgroups fill: per wave and chunk 32 + 16 MFMAs of 64 cycles and
 // 16 of 32, with three LDS round trips between them. k, q, T, P, v and the gates of the next chunk load meanwhile.
-// 2,048 tokens of the 27B layer (64 chunks): 228 us, 47 TFLOP/s; token by token (one state column in 8 lanes, DPP
+// A value, token or decay that is not finite reaches the tokens after it and the state, as token by token: a chunk with such
+// an R or Delta clears them before they meet the zeros of T and P (3 us for the tests; nothing else in a chunk without).
+// 2,048 tokens of the 27B layer (64 chunks): 231 us, 46 TFLOP/s; token by token (one state column in 8 lanes, DPP
 // sums) 781 us. Against 64 bits from the same k, q, v, beta and g, o before its rounding to bf16 is off by 7.6e-8 to 1.9e-7
 // (512 tokens, decays from e^-5 to e^-0.002 per token; 7.9e-8 to 4.3e-7 token by token, and with k . k and q . k as float32
 // chains 1.7e-7 to 2.3e-7, 10 us less in all), the state after its rounding by 1.64e-3 to 1.67e-3 in every form.
@@ -241,6 +246,8 @@ __global__ __launch_bounds__(256) void gdn_prefill_scan_kernel(const PrefillGdnA
     __shared__ __attribute__((aligned(1024))) uint8_t ring[2][2][KB];  // [stage][k, q], 16-byte chunk c of row r at c ^ (r % 16)
     __shared__ __attribute__((aligned(16))) float red[4][2][4][64][4];
     __shared__ __attribute__((aligned(16))) float sR[GC][RP], sO[GC][RP], sD[GC][RP], sW[GC][RP];
+    __shared__ int sbad[2][2];  // by chunk parity: whether an R, a Delta is not finite
+    __shared__ int sfirst[GC];  // then, by column: the first such token
     __shared__ float sf[2][3 * GC];  // beta, e^c, e^(c_last - c), by chunk parity: a chunk's tail reads while the next's are written
     const int h = blockIdx.x, grp = blockIdx.y, tid = threadIdx.x, lane = tid & 63, hf = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -283,6 +290,14 @@ __global__ __launch_bounds__(256) void gdn_prefill_scan_kernel(const PrefillGdnA
             vr[e] = a.v[((size_t)(c * GC + 8 * wave + 4 * hf + e) * Hv + h) * D + grp * 32 + (lane & 31)];
         if (tid < 3 * GC) gf = a.decay[((size_t)c * Hv + h) * 3 * GC + tid];
     };
+    // A column's R or Delta from its first token that is not finite on (at `most` by then) become zero, so that earlier
+    // tokens, whose rows of T and P multiply them by zero, stay as they are; sfirst says from where on the column is lost.
+    auto clear_from_first = [&](float(*x)[RP], int most) {
+        int first = most;
+        for (int t = most - 1; t >= 0; --t) first = finite(x[t][tid]) ? first : t;
+        for (int t = first; t < GC; ++t) x[t][tid] = 0.0f;
+        sfirst[tid] = first;
+    };
     load(0);
     for (int c = 0; c < nch; ++c) {
         // Everything but the last chunk's four output stores.
@@ -292,6 +307,7 @@ __global__ __launch_bounds__(256) void gdn_prefill_scan_kernel(const PrefillGdnA
             asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
         const float *sb = sf[c & 1], *se = sb + GC, *sw = sb + 2 * GC;
         if (tid < 3 * GC) sf[c & 1][tid] = gf;
+        if (tid < 2) sbad[c & 1][tid] = 0;
         const v4f Tc[2] = {T[0], T[1]}, Pc[2] = {P[0], P[1]};
         float vc[4];
 #pragma unroll
@@ -342,31 +358,48 @@ __global__ __launch_bounds__(256) void gdn_prefill_scan_kernel(const PrefillGdnA
             for (int w = 0; w < 4; ++w) kw[w] = *(const v4f*)red[w][0][wave][lane], qw[w] = *(const v4f*)red[w][1][wave][lane];
             __builtin_amdgcn_sched_barrier(0);
             const v4f k4 = (kw[0] + kw[1]) + (kw[2] + kw[3]), q4 = (qw[0] + qw[1]) + (qw[2] + qw[3]);
+            float zero = 0.0f;  // NaN if a value is not finite
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int t = 8 * wave + 4 * hf + e;
-                sR[t][lane & 31] = sb[t] * (vc[e] - se[t] * k4[e]);
+                const float R = sb[t] * (vc[e] - se[t] * k4[e]);
+                sR[t][lane & 31] = R;
                 sO[t][lane & 31] = se[t] * q4[e];
+                zero += 0.0f * R;
             }
+            if (zero != 0.0f) sbad[c & 1][0] = 1;
         }
         lds_barrier();
         // Delta, a 16 x 16 quarter per wave (T is lower triangular: the upper quarters sum 16 tokens).
         float rr[8];
+        auto read_r = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) rr[j] = sR[16 * (j >> 2) + 4 * lq + (j & 3)][16 * wc + lr];
+            for (int j = 0; j < 8; ++j) rr[j] = sR[16 * (j >> 2) + 4 * lq + (j & 3)][16 * wc + lr];
+        };
+        read_r();
+        const bool bad_r = __builtin_amdgcn_readfirstlane(sbad[c & 1][0]) != 0;
         __builtin_amdgcn_sched_barrier(0);
+        if (bad_r) {
+            lds_barrier();  // every wave has read
+            if (tid < GC) clear_from_first(sR, GC);
+            lds_barrier();
+            read_r();
+        }
         v4f dl = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int e = 0; e < 4; ++e) dl = mfma16(Tc[0][e], rr[e], dl);
         if (wr)
 #pragma unroll
             for (int e = 0; e < 4; ++e) dl = mfma16(Tc[1][e], rr[4 + e], dl);
+        float zero = 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int t = 16 * wr + 4 * lq + i;
             sD[t][16 * wc + lr] = dl[i];
             sW[t][16 * wc + lr] = dl[i] * sw[t];
+            zero += 0.0f * dl[i];
         }
+        if (zero != 0.0f) sbad[c & 1][1] = 1;
         const float es = se[GC - 1];
 #pragma unroll
         for (int i = 0; i < 16; ++i) S[i] *= es;
@@ -376,11 +409,21 @@ __global__ __launch_bounds__(256) void gdn_prefill_scan_kernel(const PrefillGdnA
         v4f oq;
 #pragma unroll
         for (int j = 0; j < 16; ++j) dw[j] = sW[2 * j + hf][lane & 31];
+        auto read_d = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) dd[j] = sD[16 * (j >> 2) + 4 * lq + (j & 3)][16 * wc + lr];
+            for (int j = 0; j < 8; ++j) dd[j] = sD[16 * (j >> 2) + 4 * lq + (j & 3)][16 * wc + lr];
+        };
+        read_d();
 #pragma unroll
         for (int i = 0; i < 4; ++i) oq[i] = sO[16 * wr + 4 * lq + i][16 * wc + lr];
+        const bool bad = bad_r || __builtin_amdgcn_readfirstlane(sbad[c & 1][1]) != 0;
         __builtin_amdgcn_sched_barrier(0);
+        if (bad) {
+            lds_barrier();
+            if (tid < GC) clear_from_first(sD, bad_r ? sfirst[tid] : GC);
+            lds_barrier();
+            read_d();
+        }
         v4f op[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) op[j] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
@@ -389,7 +432,15 @@ __global__ __launch_bounds__(256) void gdn_prefill_scan_kernel(const PrefillGdnA
             S = __builtin_amdgcn_mfma_f32_32x32x2f32(kt[j], dw[j], S, 0, 0, 0);
             if (j < 8) op[j >> 1] = mfma16(Pc[j >> 2][j & 3], dd[j], op[j >> 1]);
         }
-        const v4f o = oq + ((op[0] + op[1]) + (op[2] + op[3]));
+        v4f o = oq + ((op[0] + op[1]) + (op[2] + op[3]));
+        if (bad) {
+            const int from = sfirst[16 * wc + lr];
+            const bool lost = sfirst[lane & 31] < GC;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = 16 * wr + 4 * lq + i < from ? o[i] : NAN;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) S[i] = lost ? NAN : S[i];
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             a.o[((size_t)(c * GC + 16 * wr + 4 * lq + i) * Hv + h) * D + grp * 32 + 16 * wc + lr] = f2bf(o[i]);

@@ -20,6 +20,7 @@ from oracle import model as om
 from qwen38_amd import synth
 from qwen38_amd.config import LINEAR, tiny_config, with_layers
 from qwen38_amd.generate import prefill_inputs
+from qwen38_amd.quant import quantize_e4m3
 from qwen38_amd.steps import Engine, StepGraph
 from scenario import oracle_weights
 
@@ -113,3 +114,55 @@ def test_the_chunks_matrices_are_rounded_once(gpu):
     inverse = torch.linalg.inv(torch.eye(32, device="cuda", dtype=torch.float64) + (k @ k.transpose(-1, -2).contiguous()).tril(-1) * beta.unsqueeze(-1))
     # Forward substitution in float32: 32 products and sums per entry.
     assert float((pt[:, :, 0] - inverse).norm() / inverse.norm()) <= 32 * 2.0**-24
+
+
+def gdn_layer_run(change, x, n_valid):
+    """A chunk of x (row 0 from position 0) through one gated-delta layer whose weights `change` edits: output, final state."""
+    cfg = with_layers(tiny_config(1), (LINEAR,))
+    values = dict((sp.name, v) for sp, v in synth.make_all(synth.model_specs(cfg, mtp=False, head=False), 4))
+    change(values)
+    engine = Engine(cfg, 1, 1, 512, mtp=False, prefill_chunk=x.shape[1])
+    engine.load(values.items())
+    pi = prefill_inputs(cfg, 0, 0, n_valid, x.shape[1], torch.bfloat16)
+    out = StepGraph(engine)(inputs_embeds=x, **pi).cpu()[0]
+    return out, engine.gdn_state(0)["recurrent_state"].cpu()[0]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("at, n_valid", [(0, 96), (5, 96), (47, 96), (63, 96), (70, 64)])  # the last: in the padding
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_a_token_that_is_not_finite_leaves_the_earlier_ones(gpu, at, n_valid, value):
+    x = synth.hidden_states((1, 96, 1024), 4, "x")
+    want, _ = gdn_layer_run(lambda values: None, x, n_valid)
+    x[0, at] = value
+    got, state = gdn_layer_run(lambda values: None, x, n_valid)
+    assert torch.equal(got[:at], want[:at])
+    assert not bool(got[at:].isfinite().all(-1).any()) or at >= n_valid
+    assert not bool(state.isfinite().any())
+
+
+@pytest.mark.gpu
+def test_a_value_that_is_not_finite_leaves_the_other_dims(gpu):
+    """One dim of one value head, infinite at token 40 of 96: that column of the head's state is lost, every other one and
+    every earlier token's output are what they are without it."""
+    x = synth.hidden_states((1, 96, 1024), 4, "x")
+    x[..., 7] = 0.0
+    x[0, 40, 7] = 16.0
+    head, dim, name = 3, 77, "layers.0.linear_attn.in_proj_qkv"
+
+    def change(scale):
+        def edit(values):
+            row = torch.zeros(1, 1024)
+            row[0, 7] = scale
+            coded, scales = quantize_e4m3(row)
+            channel = 2 * 4 * 128 + head * 128 + dim
+            values[name][0][channel], values[name][1][channel] = coded[0], scales[0]
+
+        return edit
+
+    want, clean = gdn_layer_run(change(0.0), x, 96)
+    got, state = gdn_layer_run(change(2.0**126), x, 96)
+    assert torch.equal(got[:40], want[:40])
+    lost = torch.zeros(state.shape, dtype=torch.bool)  # [value head, key dim, value dim]
+    lost[head, :, dim] = True
+    assert torch.equal(state[~lost], clean[~lost]) and not bool(state[lost].isfinite().any())
