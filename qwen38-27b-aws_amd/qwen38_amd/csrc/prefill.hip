@@ -177,8 +177,9 @@ __global__ __launch_bounds__(256) void gdn_prefill_prep_kernel(const PrefillGdnA
                 }
             const float beta = rbf(sigmoidf_(rbf(sum[0]))) * valid;
             const float g = -expf(bf2f(a.a_log[h])) * softplusf_(rbf(sum[1]) + bf2f(a.dt_bias[h])) * valid;
-            // Summed in 64 bits: the factors are e to differences of these sums, often small ones of large ones.
-            double c = g;
+            // Summed in 64 bits: the factors are e to differences of these sums, often small ones of large ones. No term is
+            // below -200, whose e^g is zero in float32 as well, so that the differences after it keep their digits.
+            double c = g < -200.0f ? -200.0f : g;
 #pragma unroll
             for (int o = 1; o < 32; o <<= 1) {
                 const double up = __shfl_up(c, o, 32);

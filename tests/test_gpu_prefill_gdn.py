@@ -166,3 +166,40 @@ def test_a_value_that_is_not_finite_leaves_the_other_dims(gpu):
     lost = torch.zeros(state.shape, dtype=torch.bool)  # [value head, key dim, value dim]
     lost[head, :, dim] = True
     assert torch.equal(state[~lost], clean[~lost]) and not bool(state[lost].isfinite().any())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [(40,), (33, 34, 60), (0, 31, 32, 95)])
+@pytest.mark.parametrize("far", [2.0**20, 2.0**60, 2.0**100])
+def test_a_decay_to_nothing_is_one_however_far(gpu, tokens, far):
+    """e^g is zero from g = -104 down: the state restarts at such a token, and the decays after it keep their digits."""
+    x = synth.hidden_states((1, 96, 1024), 4, "x")
+    x[..., 7] = 0.0
+    x[0, list(tokens), 7] = 30.0
+
+    def change(weight):
+        def edit(values):
+            values["layers.0.linear_attn.in_proj_a"][:, 7] = weight  # times about 20: g is below -300
+            values["layers.0.linear_attn.A_log"].zero_()
+
+        return edit
+
+    want, clean = gdn_layer_run(change(16.0), x, 96)
+    got, state = gdn_layer_run(change(far), x, 96)
+    assert bool(want.isfinite().all()) and torch.equal(got, want) and torch.equal(state, clean)
+
+
+@pytest.mark.gpu
+def test_an_infinite_decay_is_a_decay_to_nothing(gpu):
+    x = synth.hidden_states((1, 96, 1024), 4, "x")
+
+    def change(log):
+        def edit(values):
+            values["layers.0.linear_attn.A_log"].fill_(log)
+            values["layers.0.linear_attn.dt_bias"].fill_(2.0)
+
+        return edit
+
+    want, clean = gdn_layer_run(change(6.0), x, 96)  # below -400 at every token
+    got, state = gdn_layer_run(change(100.0), x, 96)  # e^100 is infinite
+    assert bool(want.isfinite().all()) and torch.equal(got, want) and torch.equal(state, clean)
