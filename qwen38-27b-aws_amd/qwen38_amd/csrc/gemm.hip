@@ -878,7 +878,7 @@ hipError_t launch_stream(const GemmArgs& a0, int* splits_out, hipStream_t stream
 
 template <int TT, int NB, int EPI, bool W4>
 hipError_t dispatch_stream(const GemmArgs& a, int* splits_out, hipStream_t stream) {
-    if (a.N % 64 || a.K % 64 || a.Tpad != 32 * TT * NB || a.cus < 8 || a.cus % 8) return hipErrorInvalidValue;
+    if (a.N % 64 || a.K % 64 || a.Tpad != 32 * TT * NB || a.cus < (EPI == EPI_PARTIAL ? 1 : 8)) return hipErrorInvalidValue;
     if constexpr (EPI != EPI_PARTIAL)
         if (a.N / 64 * NB >= 2 * a.cus) return launch_stream<TT, NB, EPI, W4, 4>(a, splits_out, stream);
     return launch_stream<TT, NB, EPI, W4, 8>(a, splits_out, stream);

@@ -6,6 +6,8 @@ projection tests allow; measured about 1e-8). Finishing the split tiles by recom
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -89,6 +91,45 @@ def test_streamed_sums_of_128_tokens(gpu, k, n):
     xq = round_e5m2(x).double()
     off = (ext.fp8_linear_f32(x, *ext.pack_weight(*packed), n).double() - xq @ wd.T).abs()
     assert bool((off <= (xq.abs() @ wd.abs().T) * 2.0**-20).all())
+
+
+class GemmArgs(ctypes.Structure):
+    """csrc/kernels.h: the launcher's argument block."""
+
+    _fields_ = (
+        [(n, ctypes.c_void_p) for n in ("w", "ws", "act")] + [(n, ctypes.c_int) for n in ("K", "N", "T", "Tpad")]
+        + [("out0", ctypes.c_void_p), ("ld0", ctypes.c_int), ("n0", ctypes.c_int), ("out1", ctypes.c_void_p), ("ld1", ctypes.c_int)]
+        + [("part", ctypes.c_void_p), ("fix", ctypes.c_void_p), ("fix_floats", ctypes.c_size_t), ("counters", ctypes.c_void_p)]
+        + [(n, ctypes.c_int) for n in ("counters_n", "cus", "splits_max", "recompute", "splits", "w4", "f8")]
+    )
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [17, 64, 100])
+@pytest.mark.parametrize("cus", [8, 20, 36, 250, 255, 304])
+def test_any_number_of_cus(gpu, rows, cus):
+    """The schedule asks for no multiple of 8 compute units (a partition or another part of the chip): bf16 outputs with
+    tiles left over, and float32 sums."""
+    k, n = 1280, 4352
+    x, packed, wd = inputs(rows, k, n, False)
+    tiles, scales = ext.pack_weight(*packed)
+    scratch = ext.linear_scratch(rows, k)
+    ext.fp8_linear(x, tiles, scales, n, scratch)  # leaves x's tiles at the start of the scratch, its counters zero
+    tpad = 32 if rows <= 32 else 64 if rows <= 64 else 128
+    base, counters = scratch.data_ptr(), scratch.data_ptr() + tpad * k
+    out = torch.empty(rows, n, dtype=torch.bfloat16, device="cuda")
+    part = torch.empty(tpad, n, device="cuda")
+    a = GemmArgs(w=tiles.data_ptr(), ws=scales.data_ptr(), act=base, K=k, N=n, T=rows, Tpad=tpad, out0=out.data_ptr(), ld0=n, n0=n,
+                 part=part.data_ptr(), fix=counters + 65536 * 8, fix_floats=2 * 256 * 65536, counters=counters, counters_n=65536, cus=cus,
+                 splits_max=1)
+    launch = gpu["_Z8q38_gemmRK8GemmArgsiPiP12ihipStream_t"]
+    torch.cuda.synchronize()
+    for epi in (0, 2):
+        assert launch(ctypes.byref(a), epi, None, ctypes.c_void_p(0)) == 0
+    torch.cuda.synchronize()
+    check(out, x, wd)
+    xq = round_e5m2(x).double()
+    assert bool(((part[:rows].double() - xq @ wd.T).abs() <= (xq.abs() @ wd.abs().T) * 2.0**-20).all())
 
 
 @pytest.mark.gpu
