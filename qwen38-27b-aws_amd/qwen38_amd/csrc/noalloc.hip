@@ -1,9 +1,9 @@
 // q38_fp8_linear_noalloc: the standalone FP8 projection (q38_fp8_linear) for callers that cannot allocate device
-// memory (code under HIP graph capture, tight serving loops). Its scratch (the e5m2 input tiles, the stream-K arrival
-// counters and partial slots) is this file's static device array instead of a caller's buffer.
+// memory (code under HIP graph capture, tight serving loops). Its scratch (the e5m2 input tiles, the split tiles' arrival
+// counters and part slots) is this file's static device array instead of a caller's buffer.
 //
 // Limits: at most 64 rows (decode-sized batches), 64 x k input bytes within 2 MiB (k <= 32768), GPUs of at most 256
-// CUs. The array is 66.5 MiB; each GPU the entry point runs on holds its own copy until the process ends. Every call
+// CUs. The array is 6.5 MiB; each GPU the entry point runs on holds its own copy until the process ends. Every call
 // on one GPU shares that GPU's array: calls that overlap on one GPU race.
 
 #include <hip/hip_runtime.h>
@@ -20,9 +20,8 @@ constexpr int NOALLOC_ROWS = 64;
 constexpr int NOALLOC_CUS = 256;
 constexpr size_t NOALLOC_TILES = (size_t)2 << 20;  // e5m2 input tiles: 64 rows x 32768 inputs
 constexpr size_t NOALLOC_COUNTERS = (size_t)GEMM_COUNTERS * 8;
-// Two partial slots per CU, each the largest workgroup tile the GEMM uses at 64 rows or fewer (512 or 256 features x
-// 64 tokens over 8 waves: 32768 floats).
-constexpr size_t NOALLOC_FIX_FLOATS = (size_t)2 * NOALLOC_CUS * 32768;
+// Up to 64 rows a tile is 64 features x at most 64 tokens, and split tiles have at most one part per CU between them.
+constexpr size_t NOALLOC_FIX_FLOATS = (size_t)NOALLOC_CUS * 64 * 64;
 constexpr size_t NOALLOC_BYTES = NOALLOC_TILES + NOALLOC_COUNTERS + NOALLOC_FIX_FLOATS * 4;
 
 static __device__ __align__(256) uint8_t scratch[NOALLOC_BYTES];
@@ -69,10 +68,10 @@ int q38_fp8_linear_noalloc(const uint16_t* x, int rows, int k, const uint8_t* ti
     uint8_t* base = nullptr;
     if (scratch_on_current_device(&base)) return 1;
     hipStream_t stream = (hipStream_t)stream_;
-    // The arrival counters this call can use (one per workgroup, at most two per CU) start at zero, cleared by a kernel on
-    // the caller's stream, so a captured call records no memset.
+    // The arrival counters this call can use (one per split tile, of which there are fewer than CUs) start at zero, cleared
+    // by a kernel on the caller's stream, so a captured call records no memset.
     unsigned long long* counters = (unsigned long long*)(base + NOALLOC_TILES);
-    const int used = 2 * NOALLOC_CUS;
+    const int used = NOALLOC_CUS;
     hipLaunchKernelGGL(clear_counters_kernel, dim3((used + 255) / 256), dim3(256), 0, stream, counters, used);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return q38_report((std::string("clear_counters_kernel: ") + hipGetErrorString(e)).c_str());

@@ -32,6 +32,16 @@ def test_noalloc_projection_equals_the_scratch_argument_one_on_two_calls(gpu):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows, k, n", [(64, 2304, 8192), (33, 17408, 2048), (32, 2048, 8192), (64, 1280, 16640)])
+def test_noalloc_projection_with_every_part_slot_in_use(gpu, rows, k, n):
+    """128 tiles in two parts each, 32 in eight: as many parts as CUs, the whole array; and tiles left over beyond one a CU."""
+    tiles, words, x = packed(n, k, 7)
+    x = x[:rows].contiguous()
+    want = ext.fp8_linear(x, tiles, words, n)
+    assert torch.equal(ext.fp8_linear_noalloc(x, tiles, words, n).view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.gpu
 def test_noalloc_projection_refuses_sizes_beyond_its_array(gpu):
     tiles, words, x = packed(256, 1024, 3)
     with pytest.raises(RuntimeError, match="1 to 64 rows"):
