@@ -624,9 +624,11 @@ __global__ __launch_bounds__(WF * WT * 64, 1) void gemm_kernel(const GemmArgs a)
 // the K range and each takes all tokens (bf16 outputs from 65 tokens up: a block of 64, whose sums leave registers for the
 // loads), so nothing is shared between waves before a tile's end: weights, scales and
 // activations go straight to registers, D K-steps ahead (a K-step is 4 KiB of e4m3 weights per wave), with no ring and no
-// barrier; at the end the waves' sums are added in K order through LDS, one feature tile at a time, with the next tile's
-// first loads in flight. (With 128 to 512 features per workgroup in the ring kernel, a tile's K range was split over up
-// to twelve workgroups whose parts the last one added one after another, and every K-step met a barrier.)
+// barrier; at the end the waves' sums are added in K order through LDS, one feature tile at a time. (With 128 to 512
+// features per workgroup in the ring kernel, a tile's K range was split over up to twelve workgroups whose parts the last
+// one added one after another, and every K-step met a barrier.) For n K-steps a wave loads D + D floor(n / D): those past
+// its range, the next wave's first, are never used (12 for 10 with 5120 inputs over eight waves and D = 4; 8 for 4 where
+// 6144 inputs are split three ways).
 //
 // Schedule. What counts is that every CU moves the same bytes, and that few tiles are split. Of the tiles, whole multiples of
 // the CUs are one workgroup's each; the rest are split in K over `splits` workgroups on one XCD each, as many as the CUs

@@ -2,7 +2,8 @@
 waves, tiles left over beyond a multiple of the CUs split in K, four-wave workgroups, ragged tokens; e4m3 and MXFP4.
 
 Held against float64: half a bf16 ulp of the result for its rounding, plus 2^-20 of sum |x w| for the float32 sums (as the
-projection tests allow; measured about 1e-8). Finishing the split tiles by recomputing their parts gives the same bits."""
+projection tests allow; measured about 1e-8). Finishing the split tiles by recomputing their parts gives the same bits, in
+every form that splits."""
 
 from __future__ import annotations
 
@@ -29,7 +30,7 @@ def check(got, x, wd):
     exact, bound = xq @ wd.T, (xq.abs() @ wd.abs().T) * 2.0**-20
     ulp = torch.exp2(torch.floor(torch.log2(exact.abs().clamp_min(2.0**-126))) - 7)
     off = (got.double() - exact).abs() - bound
-    assert bool((off <= ulp * 0.5 + bound).all()), float((off / ulp).max())
+    assert bool((off <= ulp * 0.5).all()), float((off / ulp).max())
 
 
 @pytest.mark.gpu
@@ -105,12 +106,38 @@ class GemmArgs(ctypes.Structure):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("mx", [False, True])
+@pytest.mark.parametrize("rows, epi", [(17, 0), (64, 0), (100, 0), (17, 1)])
+def test_recomputed_parts_give_the_same_bits(gpu, rows, epi, mx):
+    """Finishing a split tile from its parts' sums and by computing them again (as when they ran on another XCD): bf16
+    outputs and the SwiGLU pair, e4m3 and MXFP4. 68 tiles of 64 features, split three ways (136 in blocks of 64 tokens; of
+    which, at 100 CUs, 36 are left over and split in two)."""
+    k, n = 4352, 4352
+    x, packed, _ = inputs(rows, k, n, mx)
+    tiles, scales = (ext.pack_weight_fp4 if mx else ext.pack_weight)(*packed)
+    scratch = ext.linear_scratch(rows, k)
+    (ext.mxfp4_linear if mx else ext.fp8_linear)(x, tiles, scales, n, scratch)
+    tpad = 32 if rows <= 32 else 64 if rows <= 64 else 128
+    base, counters = scratch.data_ptr(), scratch.data_ptr() + tpad * k
+    outs = [torch.zeros(rows, n, dtype=torch.bfloat16, device="cuda") if epi == 0 else torch.zeros(tpad * n // 2, dtype=torch.uint8, device="cuda") for _ in range(2)]
+    launch = gpu["_Z8q38_gemmRK8GemmArgsiPiP12ihipStream_t"]
+    torch.cuda.synchronize()
+    for recompute, out in enumerate(outs):
+        a = GemmArgs(w=tiles.data_ptr(), ws=scales.data_ptr(), act=base, K=k, N=n, T=rows, Tpad=tpad, out0=out.data_ptr(), ld0=n, n0=n,
+                     fix=counters + 65536 * 8, fix_floats=2 * 256 * 65536, counters=counters, counters_n=65536, cus=100 if rows > 64 else 256,
+                     recompute=recompute, w4=int(mx))
+        assert launch(ctypes.byref(a), epi, None, ctypes.c_void_p(0)) == 0
+    torch.cuda.synchronize()
+    assert bool((outs[0] != 0).any()) and torch.equal(outs[0].view(torch.uint8), outs[1].view(torch.uint8))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows", [17, 64, 100])
 @pytest.mark.parametrize("cus", [8, 20, 36, 250, 255, 304])
 def test_any_number_of_cus(gpu, rows, cus):
     """The schedule asks for no multiple of 8 compute units (a partition or another part of the chip): bf16 outputs with
-    tiles left over, and float32 sums."""
-    k, n = 1280, 4352
+    tiles left over and split, and float32 sums."""
+    k, n = 4352, 4352
     x, packed, wd = inputs(rows, k, n, False)
     tiles, scales = ext.pack_weight(*packed)
     scratch = ext.linear_scratch(rows, k)
