@@ -360,8 +360,11 @@ int run_mixer(q38_handle* h, int li, const StepIO& io, int rd, int wr, hipStream
         // A verify step's qkv output is also its pending input snapshot; a decode step's or a prefill chunk's goes to
         // scratch.
         uint16_t* qkv_out = io.decode || io.slot ? (uint16_t*)h->ws(h->off_qkv) : pin + wr * BKC;
-        // The gate projections (x . in_proj_b, x . in_proj_a) read only the normed input: they run on the side stream
-        // beside the qkvz GEMM, whose persistent workgroups leave room for theirs on every CU.
+        // The gate projections (x . in_proj_b, x . in_proj_a) read only the normed input. From 129 tokens up (and with the FP8
+        // MFMA) they run on the side stream beside the qkvz GEMM, whose persistent workgroups leave room for theirs on
+        // every CU. The streamed GEMM's take all of a CU's registers: beside it the gates waited for its end and the
+        // fork and join came on top (a 27B decode step of 64 rows 11.97 against 11.21 ms, 11.92 with the ring kernel and
+        // the fork; one row through a gated-delta layer 134 against 114 us).
         GatesArgs ga{};
         ga.x = (const bf16_t*)h->ws(h->off_hbf);
         ga.wb = wb;
@@ -371,7 +374,8 @@ int run_mixer(q38_handle* h, int li, const StepIO& io, int rd, int wr, hipStream
         ga.Hv = h->Hv;
         ga.groups = h->gate_groups;
         ga.part = (float*)h->ws(h->off_gates);
-        const bool fork = h->side_stream != nullptr;
+        const bool streamed = h->Tpad <= 128 && (fp4_layer(h, li) || h->cfg.projection_mfma != Q38_MFMA_FP8);
+        const bool fork = h->side_stream != nullptr && !streamed;
         if (fork) {
             HIP_TRY(hipEventRecord(h->fork_ev, stream));
             HIP_TRY(hipStreamWaitEvent(h->side_stream, h->fork_ev, 0));
