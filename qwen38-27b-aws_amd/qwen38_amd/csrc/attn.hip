@@ -464,8 +464,8 @@ __global__ __launch_bounds__(SW * 64) void attn_fused_kernel(const AttnArgs a) {
 // that is the wave's own, so there is no barrier: copied a KB of contiguous cache per instruction, read back per lane
 // without bank conflicts (16-byte piece c of row r lies at c ^ r). Each lane carries the maximum and the sum of e^(s - max)
 // over its own positions of its query row; the four lanes of a row merge theirs at the chunk's end.
-// 16 x 4 heads of 28,672 positions on average, 24 query rows: 213 us (0.94 GB of keys, 88 MB of scores, 4.8 TB/s); 64 x 4
-// heads of 7,168, FP8, 6 query rows: 110 us (0.47 GB, 4.3 TB/s). Before, as sixteen waves of 32 positions each around two
+// 16 x 4 heads of 28,672 positions on average, 24 query rows: 224 us (0.94 GB of keys, 88 MB of scores, 4.6 TB/s); 64 x 4
+// heads of 7,168, FP8, 6 query rows: 115 us (0.47 GB, 4.1 TB/s); 213 and 110 where the following were measured. As sixteen waves of 32 positions each around two
 // barriers, 231 and 157 us; with keys read straight into operand registers 251 and 129 us (every load touches 64 cache
 // lines, and the CU's line rate, not HBM, sets the pace); 32 positions at a time, which leaves room for one wave per SIMD,
 // 218 and 135 us; with each block's scores stored at once 235 and 112 us.
@@ -931,8 +931,10 @@ hipError_t launch_attn(AttnArgs a, hipStream_t stream) {
         while (ns > 1 && (size_t)pairs * ns * QT * 8192 > a.pv_part_floats) --ns;
         a.pv_splits = ns;
         // Positions per wave of attn_scores: 512, fewer while that leaves less than three rounds of the eight waves a CU
-        // holds (over the whole cache: the rows' own lengths are on the device), so that the last round is a short one:
-        // scores and weights x V 202 + 117 us with 256 against 221 + 117 with 512 at the shapes above.
+        // holds (over the whole cache: the rows' own lengths are on the device), so that the last round is a short one: a
+        // decode layer of 8 rows of 16K positions 235 against 250 us with 512 throughout, a verify layer of 16 rows of 8K 267
+        // against 282. At the shapes above, where 256 are taken, the two are equal (scores + weights x V 224 + 211 against
+        // 226 + 206, 115 + 105 against 117 + 102).
         a.chunk = ATTN_CHUNK;
         while (a.chunk > ATTN_CHUNK_MIN && pairs * ((a.S + a.chunk - 1) / a.chunk) < 24L * a.cus) a.chunk /= 2;
         a.nchunks = (a.S + a.chunk - 1) / a.chunk;

@@ -47,10 +47,10 @@ struct PlanesArgs {
 // A workgroup of KW waves takes 32 FR features x 32 TT tokens; its waves split K and add up through LDS at the end, a feature
 // tile and a parity at a time, so nothing is shared before that: every operand goes straight to registers, D K-steps
 // ahead, without a barrier. Bound by the L2 at 64 tokens per block (FR = 4: 12 KB per K-step for 32 MFMAs), by HBM's
-// weights and the launches at few tokens. With the tiles' preparation, 200 rows of 5120 -> 5120 take 25.4 us (0.41 PFLOP/s),
-// 1,024 of 5120 -> 14336 175 us (0.86 PFLOP/s); as a projection per parity, the other parity's inputs zero, in 256 x 256
-// tiles, the former took 148 us. Without the scheduling barrier the compiler moves the 128 x 64 tile's loads to their
-// use (31.4 against 25.4 us).
+// weights and the launches at few tokens. With the tiles' preparation, 200 rows of 5120 -> 5120 take 22.5 us a call among
+// others (0.47 PFLOP/s), 1,024 of 5120 -> 14336 176 us (0.85 PFLOP/s); as a projection per parity, the other parity's inputs
+// zero, in 256 x 256 tiles, they took 148 and 287 us. Without the scheduling barrier the compiler moves the 128 x 64
+// tile's loads to their use (31.4 against 25.4 us in a sweep that waited for each call).
 template <int FR, int TT, int KW, int D>
 __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(KW / 4))) void fp4_planes_kernel(const PlanesArgs a) {
     constexpr int G = TT * 4, GW = (G + KW - 1) / KW;  // (token tile, quarter of the rows) quads of a feature tile, per wave
