@@ -20,9 +20,9 @@
 //   attn_prefill_max, attn_prefill, attn_prefill_finish: blocked_attention (model.py:170-191) over the row's cached
 //                      positions before `start` and the chunk's own tokens causally, in the reference's blocks of 2048
 //                      positions of [cache, chunk]: per block the running max, e^(s - max) summed in float32, the
-//                      weights in bf16 times V on the MFMA with float32 sums, output and sum rescaled across blocks;
-//                      then out / sum, the gate, e5m2. Positions a row cannot see are skipped: the reference gives them
-//                      weights of exactly zero.
+//                      weights in bf16 times V on the MFMA (float32 sums, rounded to bf16 once per block, as the
+//                      reference's bf16 matmul), output and sum rescaled across blocks; then out / sum, the gate, e5m2.
+//                      Positions a row cannot see are skipped: the reference gives them weights of exactly zero.
 #include <algorithm>
 #include <type_traits>
 
